@@ -232,6 +232,12 @@ int isoext_mc_dense_keyed(const float *values, const int64_t shape[3], const flo
 int isoext_mc_backward(const isoext_grid *g, float level, const float *grad_v, const int64_t *vertex_src,
                        int64_t nv, float *grad_values, void *stream);
 
+/* Backward of sparse marching cubes from the vsrc and vjac of
+ * isoext_mc_sparse_run: writes the whole (n_sparse, 8) gradient, zero rows
+ * included (grad_values need not be cleared). */
+int isoext_mc_sparse_backward(int64_t n_sparse, const float *grad_v, const int64_t *vsrc, const float *vjac,
+                              int64_t nv, float *grad_values, void *stream);
+
 /* Benchmark input generation (no reference counterpart; the reference's SDFs
  * are torch code, src/isoext/sdf.py): out[x,y,z] = min_k |p - c_k| - r_k over
  * k <= 256 spheres given as device float4 (cx, cy, cz, r). */
@@ -296,6 +302,23 @@ int isoext_mc_sparse_count(const isoext_grid *g, float level, int64_t *scratch, 
 int isoext_mc_sparse(const isoext_grid *g, float level, int method, int64_t ninst, void *workspace,
                      int64_t workspace_bytes, float *out_v, int64_t cap_v, int32_t *out_f,
                      int64_t cap_f, int64_t *vsrc, int64_t counts[2], void *stream);
+
+/* The same in two steps that find the cases of the cells once: the first
+ * leaves them in `scratch` (isoext_mc_sparse_scratch_bytes(n) bytes, 16-byte
+ * aligned) and returns counts = {crossing-edge instances, active cells}, the
+ * second takes both (the grid and level unchanged between the two) and a
+ * workspace of isoext_mc_sparse_run_bytes(instances, active cells) bytes,
+ * 16-byte aligned.  vsrc comes out ascending; vjac (optional, two floats a
+ * vertex, 8-byte aligned) receives the derivatives of the vertex's coordinate
+ * along its edge by the edge's two end values.  Both synchronise. */
+int64_t isoext_mc_sparse_scratch_bytes(int64_t n);
+int64_t isoext_mc_sparse_run_bytes(int64_t ninst, int64_t nact);
+int isoext_mc_sparse_cases(const isoext_grid *g, float level, void *scratch, int64_t scratch_bytes,
+                           int64_t counts[2], void *stream);
+int isoext_mc_sparse_run(const isoext_grid *g, float level, int method, const void *scratch,
+                         const int64_t case_counts[2], void *workspace, int64_t workspace_bytes, float *out_v,
+                         int64_t cap_v, int32_t *out_f, int64_t cap_f, int64_t *vsrc, float *vjac,
+                         int64_t counts[2], void *stream);
 
 /* ---- captured plans (no reference counterpart: repeated extractions of one
  * grid buffer, e.g. an optimisation loop that updates the values in place) ----

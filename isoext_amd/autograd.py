@@ -32,6 +32,9 @@ from .sparse import SparseGrid, mc_sparse
 _lib.declare("isoext_mc_backward", ctypes.c_int, [ctypes.POINTER(IsoGrid), ctypes.c_float, ctypes.c_void_p,
                                                   ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p,
                                                   ctypes.c_void_p])
+_lib.declare("isoext_mc_sparse_backward", ctypes.c_int, [ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p,
+                                                         ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p,
+                                                         ctypes.c_void_p])
 
 
 class _View:
@@ -58,31 +61,40 @@ class MarchingCubesFunction(torch.autograd.Function):
         if isinstance(grid, UniformGrid):
             v, f, info = mc_dense_raw(vals, grid.shape, grid.aabb_min, grid.aabb_max, level, method,
                                       want_keys=True)
-            src = info["keys"]
+            src, jac = info["keys"], None
         else:
-            v, f, src = mc_sparse(view, level, method, want_src=True)
+            v, f, src, jac = mc_sparse(view, level, method, want_jac=True)
             if v is None:
                 v = torch.empty((0, 3), dtype=torch.float32, device=vals.device)
                 f = torch.empty((0, 3), dtype=torch.int32, device=vals.device)
                 src = torch.empty(0, dtype=torch.int64, device=vals.device)
+                jac = torch.empty((0, 2), dtype=torch.float32, device=vals.device)
         ctx.view = view
         ctx.level = float(level)
-        ctx.save_for_backward(vals, src)
+        ctx.save_for_backward(vals, src, jac)
         ctx.mark_non_differentiable(f)
+        ctx.set_materialize_grads(False)   # no gradient of the faces is made up
         return v, f
 
     @staticmethod
     def backward(ctx, grad_v, grad_f):
-        vals, src = ctx.saved_tensors
-        grad = torch.zeros_like(vals)
-        if grad_v is not None and src.numel():
-            gv = grad_v.contiguous().float()
-            g = grid_struct(ctx.view)
-            dev = vals.device
-            with torch.cuda.device(dev):
-                _lib.check(_lib.lib().isoext_mc_backward(ctypes.byref(g), ctx.level, gv.data_ptr(), src.data_ptr(),
-                                                         src.numel(), grad.data_ptr(), _lib.stream_ptr(dev)),
-                           "marching_cubes backward")
+        vals, src, jac = ctx.saved_tensors
+        if grad_v is None or not src.numel():
+            return torch.zeros_like(vals), None, None, None
+        L = _lib.lib()
+        gv = grad_v.contiguous().float()
+        dev = vals.device
+        with torch.cuda.device(dev):
+            if jac is not None:   # sparse: every row of the gradient is written
+                grad = torch.empty_like(vals)
+                rc = L.isoext_mc_sparse_backward(vals.shape[0], gv.data_ptr(), src.data_ptr(), jac.data_ptr(),
+                                                 src.numel(), grad.data_ptr(), _lib.stream_ptr(dev))
+            else:
+                grad = torch.zeros_like(vals)
+                g = grid_struct(ctx.view)
+                rc = L.isoext_mc_backward(ctypes.byref(g), ctx.level, gv.data_ptr(), src.data_ptr(), src.numel(),
+                                          grad.data_ptr(), _lib.stream_ptr(dev))
+        _lib.check(rc, "marching_cubes backward")
         return grad, None, None, None
 
 

@@ -78,6 +78,66 @@ __global__ void k_bwd_sparse(const float *grad_v, const int64_t *vsrc, int64_t n
     if (gb != 0.0f) atomicAdd(&grad_values[8 * slot + cb], gb);
 }
 
+// A workgroup owns kRows rows of the gradient: its vertices are one run of
+// the ascending vsrc, and a row's vertices (its cell's representatives) are
+// consecutive, so the first of them adds up the row in LDS without atomics,
+// and every row leaves as one coalesced write.  Bound by that write (32 B a
+// cell); with the derivatives from the forward pass the vertices' values and
+// ids, scattered over most lines of the grid's arrays, are not read again.
+// A scatter by atomics into a cleared array touches nearly every line of it
+// three times.
+constexpr int kRows = 512;
+
+// The runs' bounds, left in the first row that each workgroup will write
+// (found by one lane each: a search inside the workgroup costs it a chain of
+// loads, and a wave-wide one fetches more lines than the vertices take).
+__global__ void __launch_bounds__(64) k_bwd_sparse_runs(const int64_t *vsrc, int64_t nv, int64_t n,
+                                                        float *grad_values) {
+    const int64_t b = (int64_t) blockIdx.x * 63 + threadIdx.x, s0 = b * kRows;
+    int64_t r[2];   // a run ends where the next lane's begins: 63 runs a wave
+    r[0] = lower_bound8(vsrc, nv, 12 * s0);
+    r[1] = __shfl_down(r[0], 1);
+    if (threadIdx.x == 63 || s0 >= n) return;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        grad_values[8 * s0 + k] = __int_as_float((int) (r[k >> 1] >> (32 * (k & 1))));
+}
+
+__global__ void __launch_bounds__(kB) k_bwd_sparse_rows(const float *grad_v, const int64_t *vsrc, const float2 *vjac,
+                                                        int64_t n, float *grad_values) {
+    __shared__ float row[8 * kRows];
+    const int64_t s0 = (int64_t) blockIdx.x * kRows;
+    const int tid = threadIdx.x;
+    uint32_t r4[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) r4[k] = (uint32_t) __float_as_int(grad_values[8 * s0 + k]);
+    const int64_t lo = (int64_t) ((uint64_t) r4[1] << 32 | r4[0]), hi = (int64_t) ((uint64_t) r4[3] << 32 | r4[2]);
+    for (int k = tid; k < 8 * kRows; k += kB) row[k] = 0.0f;
+    __syncthreads();
+    for (int64_t i = lo + tid; i < hi; i += kB) {
+        int src = (int) (vsrc[i] - 12 * s0);
+        const int r = src / 12;
+        if (i > lo && (int) (vsrc[i - 1] - 12 * s0) / 12 == r) continue;   // not its row's first
+        for (int64_t j = i;;) {
+            const int e = src - 12 * r, ax = edge_axis(e);
+            const float g[3] = {grad_v[3 * j], grad_v[3 * j + 1], grad_v[3 * j + 2]};
+            // the edge is along one axis; a gradient that is not finite anywhere counts for nothing
+            const float s = (ax == 0 ? g[0] : (ax == 1 ? g[1] : g[2])) + (0.0f * g[0] + 0.0f * g[1] + 0.0f * g[2]);
+            const float2 d = vjac[j];
+            const float ga = s * d.x, gb = s * d.y;
+            if (isfinite(ga)) row[8 * r + edge_a(e)] += ga;
+            if (isfinite(gb)) row[8 * r + edge_b(e)] += gb;
+            if (++j >= hi) break;
+            src = (int) (vsrc[j] - 12 * s0);
+            if (src / 12 != r) break;
+        }
+    }
+    __syncthreads();
+    float *out = grad_values + 8 * s0;
+    const int m = (int) min<int64_t>(kRows, n - s0) * 8;
+    for (int k = tid; k < m; k += kB) __builtin_nontemporal_store(row[k], out + k);
+}
+
 }   // namespace
 
 hipError_t mc_backward_dense(const float *grad_v, const int64_t *keys, int64_t nv, const float *values,
@@ -94,6 +154,14 @@ hipError_t mc_backward_sparse(const float *grad_v, const int64_t *vsrc, int64_t 
     if (nv == 0) return hipSuccess;
     hipLaunchKernelGGL(k_bwd_sparse, dim3((unsigned) ((nv + kB - 1) / kB)), dim3(kB), 0, st, grad_v, vsrc, nv,
                        values, ids, g, level, grad_values);
+    return hipGetLastError();
+}
+
+hipError_t mc_backward_sparse_rows(const float *grad_v, const int64_t *vsrc, const float2 *vjac, int64_t nv, int64_t n,
+                                   float *grad_values, hipStream_t st) {
+    const int64_t nblk = (n + kRows - 1) / kRows;
+    hipLaunchKernelGGL(k_bwd_sparse_runs, dim3((unsigned) ((nblk + 62) / 63)), dim3(64), 0, st, vsrc, nv, n, grad_values);
+    hipLaunchKernelGGL(k_bwd_sparse_rows, dim3((unsigned) nblk), dim3(kB), 0, st, grad_v, vsrc, vjac, n, grad_values);
     return hipGetLastError();
 }
 

@@ -1455,6 +1455,15 @@ int64_t isoext_mc_sparse_workspace_bytes(int64_t n, int64_t ninst) {
     return (int64_t) iso::sparse_mc_work_bytes(n, ninst);
 }
 
+// weld_cand_eps for a sparse grid, whose axes may be far longer than a dense
+// one's: its walk over an axis up to 2^16 points, beyond that every cell goes
+// by position (the walk would cost more than it saves).
+static float sparse_cand_eps(const int64_t shape[3], const float *amin, const float *amax) {
+    for (int a = 0; a < 3; ++a)
+        if (shape[a] > (1 << 16)) return INFINITY;
+    return weld_geom(shape, amin, amax).cand_eps;
+}
+
 static iso::SparseMcIn smc_in(const isoext_grid *g, float level, int method) {
     iso::SparseMcIn in;
     in.values = g->values;
@@ -1463,7 +1472,57 @@ static iso::SparseMcIn smc_in(const isoext_grid *g, float level, int method) {
     in.g = geom_of(g->shape, g->aabb_min, g->aabb_max);
     in.level = level;
     in.method = method;
+    in.cand_eps = sparse_cand_eps(g->shape, g->aabb_min, g->aabb_max);
+    const int64_t cx = g->shape[0] - 1, cy = g->shape[1] - 1, cz = g->shape[2] - 1;
+    if (cx > 0 && cy > 0 && cz > 0 && cx < (1ll << 31) && cy < (1ll << 31) && cz < (1ll << 31) &&
+        cx * cy < (1ll << 31) && cx * cy < (1ll << 52) / cz) {
+        in.div.inv_cz = 1.0 / (double) cz;
+        in.div.cy = iso::UDiv32((uint32_t) cy);
+        in.div.ncell = cx * cy * cz;
+    }
     return in;
+}
+
+int64_t isoext_mc_sparse_scratch_bytes(int64_t n) { return n > 0 ? (int64_t) iso::sparse_mc_scratch_bytes(n) : 0; }
+
+int64_t isoext_mc_sparse_run_bytes(int64_t ninst, int64_t nact) {
+    return ninst > 0 && nact > 0 ? (int64_t) iso::sparse_mc_run_bytes(ninst, nact) : 0;
+}
+
+int isoext_mc_sparse_cases(const isoext_grid *g, float level, void *scratch, int64_t scratch_bytes,
+                           int64_t counts[2], void *stream) {
+    counts[0] = counts[1] = 0;
+    AABB_CHECK(g->aabb_min, g->aabb_max);
+    if (!g->sparse_cell_ids || g->n_sparse == 0) return ISOEXT_OK;
+    if (scratch_bytes < isoext_mc_sparse_scratch_bytes(g->n_sparse))
+        return fail(ISOEXT_E_WORKSPACE, "sparse marching cubes scratch too small");
+    HIP_CHECK(iso::sparse_mc_cases(smc_in(g, level, 0), scratch, counts[0], counts[1], (hipStream_t) stream),
+              "sparse cases");
+    return ISOEXT_OK;
+}
+
+int isoext_mc_sparse_run(const isoext_grid *g, float level, int method, const void *scratch,
+                         const int64_t case_counts[2], void *workspace, int64_t workspace_bytes, float *out_v,
+                         int64_t cap_v, int32_t *out_f, int64_t cap_f, int64_t *vsrc, float *vjac,
+                         int64_t counts[2], void *stream) {
+    counts[0] = counts[1] = 0;
+    if (method != 0 && method != 1) return fail(ISOEXT_E_ARG, "Unknown method: %d", method);
+    AABB_CHECK(g->aabb_min, g->aabb_max);
+    const int64_t ninst = case_counts[0], nact = case_counts[1];
+    if (!g->sparse_cell_ids || g->n_sparse == 0 || ninst == 0) return ISOEXT_OK;
+    if (workspace_bytes < isoext_mc_sparse_run_bytes(ninst, nact))
+        return fail(ISOEXT_E_WORKSPACE, "sparse marching cubes workspace too small");
+    iso::SparseMcOut o{out_v, out_v ? cap_v : 0, out_f, out_f ? cap_f : 0, vsrc, (float2 *) vjac};
+    int64_t nv = 0, nf = 0;
+    HIP_CHECK(iso::sparse_mc_run(smc_in(g, level, method), scratch, ninst, nact, workspace, (size_t) workspace_bytes, o,
+                                 nv, nf, (hipStream_t) stream),
+              "sparse marching cubes");
+    counts[0] = nv;
+    counts[1] = nf;
+    if (nv > cap_v || nf > cap_f)
+        return fail(ISOEXT_E_CAPACITY, "output capacity too small: need %lld vertices, %lld faces", (long long) nv,
+                    (long long) nf);
+    return ISOEXT_OK;
 }
 
 int isoext_mc_sparse_count(const isoext_grid *g, float level, int64_t *scratch, int64_t *ninst, void *stream) {
@@ -1496,6 +1555,15 @@ int isoext_mc_sparse(const isoext_grid *g, float level, int method, int64_t nins
     return ISOEXT_OK;
 }
 
+
+int isoext_mc_sparse_backward(int64_t n_sparse, const float *grad_v, const int64_t *vsrc, const float *vjac, int64_t nv,
+                              float *grad_values, void *stream) {
+    if (n_sparse <= 0) return ISOEXT_OK;
+    HIP_CHECK(iso::mc_backward_sparse_rows(grad_v, vsrc, (const float2 *) vjac, nv, n_sparse, grad_values,
+                                           (hipStream_t) stream),
+              "sparse marching cubes backward");
+    return ISOEXT_OK;
+}
 
 int isoext_mc_backward(const isoext_grid *g, float level, const float *grad_v, const int64_t *vertex_src, int64_t nv,
                        float *grad_values, void *stream) {

@@ -56,6 +56,38 @@ __device__ __forceinline__ int wave_incl_max(int v) {
     return wave_incl_scan(v, [](int a, int b) { return a > b ? a : b; });
 }
 
+// First index of ascending a[0, n) with a value >= key.  Seven probes a step
+// (independent loads) make a third of a binary search's dependent steps.
+__device__ __forceinline__ int64_t lower_bound8(const int64_t *a, int64_t n, int64_t key) {
+    int64_t lo = 0, len = n;
+    while (len > 0) {
+        const int64_t step = (len + 7) >> 3;   // probes at the ends of eight parts
+        int c = 0;
+#pragma unroll
+        for (int j = 1; j < 8; ++j) {
+            const int64_t q = step * j;
+            c += (q <= len && a[lo + min(q, len) - 1] < key) ? 1 : 0;
+        }
+        // the first c parts are below key, the answer in part c (or at its end)
+        lo += step * c;
+        len = min(step, len - step * c);
+        if (step == 1) {   // one entry is left
+            if (len > 0 && a[lo] < key) ++lo;
+            break;
+        }
+    }
+    return lo;
+}
+
+// Workgroups go to the 8 XCDs in turn, and each XCD has an L2 of its own: for
+// work items whose neighbours share data, workgroup b of n takes item
+// xcd_item(b, n), so that each XCD sweeps one contiguous eighth of them.  The
+// grid is 8 * ceil(n / 8) workgroups at least; a result >= n has no item.
+__device__ __forceinline__ int64_t xcd_item(int64_t b, int64_t n) {
+    const int64_t per = (n + 7) >> 3, i = b >> 3;
+    return i < per ? (b & 7) * per + i : n;
+}
+
 ISO_HD int32_t f2i_bits(float f) {
     union {
         float f;

@@ -5,11 +5,20 @@
 
 #include <algorithm>
 
+#include "common.h"
+
 namespace iso {
 
 struct SparseGeom {
     int64_t X, Y, Z;   // points per axis
     float amin[3], amax[3];
+};
+
+// Reciprocals of the cells per axis; ncell = 0: not used.
+struct SparseDiv {
+    double inv_cz = 0.0;
+    UDiv32 cy;
+    int64_t ncell = 0;
 };
 
 struct SparseMcIn {
@@ -19,18 +28,23 @@ struct SparseMcIn {
     SparseGeom g;
     float level;
     int method;
+    float cand_eps;   // bound on t (or 1 - t) of a vertex within 16 ulps of a grid point
+    SparseDiv div;
 };
 
+// Active cells (in id order) and crossing-edge instances (cell by cell, in
+// edge order) of a run.
 struct SparseMcWork {
-    uint32_t *cst;        // per cell: crossing-edge mask (bits 0-11), case index (bits 16-23)
-    int64_t *cell_inst;   // first instance of each active cell
-    int32_t *inst_cell;   // cell slot of each instance
-    float *ipos;          // instance positions
-    int64_t *isrc;        // slot * 12 + edge of each instance
-    int64_t *rkey;        // instance index of its representative (first instance at its position)
-    uint8_t *used;        // the representative is a corner of a kept face
-    int32_t *vid;         // vertex id of the instance's representative
-    int *err;
+    int64_t *aid;      // per active cell: dense cell id
+    int32_t *aslot;    // its slot
+    uint2 *ainfo;      // its first instance; case, special flag, crossing edges
+    uint32_t *ares;    // edges that represent themselves, kept faces, special flag
+    uint32_t *alook;   // edges whose vertex may lie near a grid point
+    int32_t *win;      // per workgroup: the runs of active cells its cells' lower neighbours are in
+    int64_t *bid;      // first id of each workgroup's active cells
+    int32_t *rkey;     // per instance: its representative (first instance at its position)
+    int32_t *vid;      // vertex id of a representative
+    uint8_t *used;     // special cells: the representative is a corner of a kept face
 };
 
 struct SparseMcOut {
@@ -39,6 +53,7 @@ struct SparseMcOut {
     int32_t *f;
     int64_t cap_f;
     int64_t *vsrc;   // optional: slot * 12 + edge of each output vertex
+    float2 *vjac = nullptr;   // optional: derivatives of its coordinate along the edge by the edge's end values
 };
 
 hipError_t sparse_corner_points(const int64_t *ids, int64_t n, const SparseGeom &g, float *out, hipStream_t st);
@@ -53,6 +68,17 @@ hipError_t sparse_setop(const int64_t *a, int64_t na, const int64_t *b, int64_t 
 hipError_t sparse_gather_rows(const float *old_values, const int64_t *slot, int64_t n, float dflt, float *out,
                               hipStream_t st);
 hipError_t sparse_crossing_flags(const float *values, int64_t n, float level, uint8_t *flags, hipStream_t st);
+// Marching cubes in two steps: the cases of all cells (scratch of
+// sparse_mc_scratch_bytes(n), kept for the second step; synchronises for the
+// counts), then the run (work of sparse_mc_run_bytes; synchronises for the
+// mesh sizes).
+size_t sparse_mc_scratch_bytes(int64_t n);
+size_t sparse_mc_run_bytes(int64_t ninst, int64_t nact);
+hipError_t sparse_mc_cases(const SparseMcIn &in, void *scratch, int64_t &ninst, int64_t &nact, hipStream_t st);
+hipError_t sparse_mc_run(const SparseMcIn &in, const void *scratch, int64_t ninst, int64_t nact, void *work,
+                         size_t work_bytes, SparseMcOut &o, int64_t &nv, int64_t &nf, hipStream_t st);
+// The same with nothing kept between the count and the run (the cases are
+// found twice): scratch of the count 8 * (n / 256 + 16) bytes.
 size_t sparse_mc_work_bytes(int64_t n, int64_t ninst);
 hipError_t sparse_mc_count(const SparseMcIn &in, int64_t *scratch, int64_t &ninst, hipStream_t st);
 hipError_t sparse_mc(const SparseMcIn &in, int64_t ninst, void *work, size_t work_bytes, SparseMcOut &o,

@@ -32,7 +32,11 @@ from .grid import FLT_MAX, Grid, _shape3, _vec3, check_cuda_f32
 vp, i64, f32 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_float
 _lib.declare("isoext_sparse_corner_points", ctypes.c_int, [vp, i64, _lib.I64x3, _lib.F32x3, _lib.F32x3, vp, vp])
 _lib.declare("isoext_sparse_crossing_flags", ctypes.c_int, [vp, i64, f32, vp, vp])
-_lib.declare("isoext_mc_sparse_workspace_bytes", i64, [i64, i64])
+_lib.declare("isoext_mc_sparse_scratch_bytes", i64, [i64])
+_lib.declare("isoext_mc_sparse_run_bytes", i64, [i64, i64])
+_lib.declare("isoext_mc_sparse_cases", ctypes.c_int, [vp, f32, vp, i64, i64 * 2, vp])
+_lib.declare("isoext_mc_sparse_run", ctypes.c_int, [vp, f32, ctypes.c_int, vp, i64 * 2, vp, i64, vp, i64, vp, i64, vp,
+                                                    vp, i64 * 2, vp])
 _lib.declare("isoext_sparse_setop_scratch_bytes", i64, [i64, i64])
 _lib.declare("isoext_sparse_union", ctypes.c_int, [vp, i64, vp, i64, vp, i64, vp, vp, vp, vp])
 _lib.declare("isoext_sparse_difference", ctypes.c_int, [vp, i64, vp, i64, vp, i64, vp, vp, vp, vp])
@@ -218,34 +222,39 @@ def grid_struct_of(grid):
     return grid_struct(grid)
 
 
-def mc_sparse(grid: SparseGrid, level: float, method: int, want_src: bool = False):
-    """Marching cubes over a sparse grid; returns (v, f[, vsrc])."""
+def mc_sparse(grid: SparseGrid, level: float, method: int, want_src: bool = False, want_jac: bool = False):
+    """Marching cubes over a sparse grid; returns (v, f[, vsrc[, vjac]]):
+    vsrc the slot * 12 + edge of each vertex, vjac ((V, 2) float32) the
+    derivatives of its coordinate along that edge by the edge's end values."""
     L = _lib.lib()
     dev = grid.device
     n = grid.get_num_cells()
-    empty = (None, None, None) if want_src else (None, None)
+    empty = (None,) * (4 if want_jac else 3 if want_src else 2)
     if n == 0:
         return empty
     g = grid_struct_of(grid)
-    scratch = workspace.get("sparse_count", 8 * (n // 256 + 32), dev)
-    ninst = ctypes.c_int64(0)
+    nbytes = L.isoext_mc_sparse_scratch_bytes(n)
+    scratch = workspace.get("sparse_cases", nbytes, dev)
+    case_counts = (ctypes.c_int64 * 2)()
     with torch.cuda.device(dev):
         stream = _lib.stream_ptr(dev)
-        _lib.check(L.isoext_mc_sparse_count(ctypes.byref(g), float(level), scratch.data_ptr(), ctypes.byref(ninst),
-                                            stream), "marching_cubes")
-        ni = int(ninst.value)
+        _lib.check(L.isoext_mc_sparse_cases(ctypes.byref(g), float(level), scratch.data_ptr(), scratch.numel(),
+                                            case_counts, stream), "marching_cubes")
+        ni, na = int(case_counts[0]), int(case_counts[1])
         if ni == 0:
             return empty
-        ws = workspace.get("sparse_mc", L.isoext_mc_sparse_workspace_bytes(n, ni), dev)
-        cap_v, cap_f = ni, 5 * n
+        ws = workspace.get("sparse_mc", L.isoext_mc_sparse_run_bytes(ni, na), dev)
+        cap_v, cap_f = ni, 5 * na
         counts = (ctypes.c_int64 * 2)()
         for _ in range(2):
             v = torch.empty((max(cap_v, 1), 3), dtype=torch.float32, device=dev)
             f = torch.empty((max(cap_f, 1), 3), dtype=torch.int32, device=dev)
-            src = torch.empty(max(cap_v, 1), dtype=torch.int64, device=dev) if want_src else None
-            rc = L.isoext_mc_sparse(ctypes.byref(g), float(level), int(method), ni, ws.data_ptr(), ws.numel(),
-                                    v.data_ptr(), cap_v, f.data_ptr(), cap_f,
-                                    src.data_ptr() if src is not None else None, counts, stream)
+            src = torch.empty(max(cap_v, 1), dtype=torch.int64, device=dev) if want_src or want_jac else None
+            jac = torch.empty((max(cap_v, 1), 2), dtype=torch.float32, device=dev) if want_jac else None
+            rc = L.isoext_mc_sparse_run(ctypes.byref(g), float(level), int(method), scratch.data_ptr(), case_counts,
+                                        ws.data_ptr(), ws.numel(), v.data_ptr(), cap_v, f.data_ptr(), cap_f,
+                                        src.data_ptr() if src is not None else None,
+                                        jac.data_ptr() if jac is not None else None, counts, stream)
             if rc == _lib.E_CAPACITY:
                 cap_v, cap_f = int(counts[0]), int(counts[1])
                 continue
@@ -255,6 +264,8 @@ def mc_sparse(grid: SparseGrid, level: float, method: int, want_src: bool = Fals
     if nf == 0:
         return empty
     v, f = v[:nv], f[:nf]
+    if want_jac:
+        return v, f, src[:nv], jac[:nv]
     if want_src:
         return v, f, src[:nv]
     return v, f
