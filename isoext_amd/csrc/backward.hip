@@ -85,12 +85,14 @@ __global__ void k_bwd_sparse(const float *grad_v, const int64_t *vsrc, int64_t n
 // cell); with the derivatives from the forward pass the vertices' values and
 // ids, scattered over most lines of the grid's arrays, are not read again.
 // A scatter by atomics into a cleared array touches nearly every line of it
-// three times.
+// three times: 0.66 ms and 0.12 ms for the clearing at 25.7 M cells and 9.7 M
+// vertices, against 0.21 ms (1.09 GB, 5.2 TB/s) and 0.03 ms for the runs.
+// kRows 1024 (a longer chain per workgroup, half the wavefronts): 0.32 ms.
 constexpr int kRows = 512;
 
 // The runs' bounds, left in the first row that each workgroup will write
 // (found by one lane each: a search inside the workgroup costs it a chain of
-// loads, and a wave-wide one fetches more lines than the vertices take).
+// loads, and a wave-wide one fetched as many lines as the vertices take).
 __global__ void __launch_bounds__(64) k_bwd_sparse_runs(const int64_t *vsrc, int64_t nv, int64_t n,
                                                         float *grad_values) {
     const int64_t b = (int64_t) blockIdx.x * 63 + threadIdx.x, s0 = b * kRows;
