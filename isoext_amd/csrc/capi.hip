@@ -315,8 +315,8 @@ bool grid_has_cells(const isoext_grid *g) {
 }
 
 struct DcLayout {
-    size_t o_dual, o_cond, o_cnt, o_used, o_bnd, o_qn, o_qm, o_bsum, o_part, o_tot, o_tri, o_hs, o_hm, o_rep, o_fin,
-        o_ak, o_av, total;
+    size_t o_dual, o_cond, o_used, o_bnd, o_qn, o_qm, o_bsum, o_part, o_tot, o_tri, o_hs, o_rep, o_fin, o_ak, o_av,
+        total;
     int64_t hslots;
 };
 
@@ -334,7 +334,6 @@ DcLayout dc_layout(int64_t ncells, int64_t npts) {
     };
     L.o_dual = take(sizeof(float) * 3 * std::max<int64_t>(ncells, 1));
     L.o_cond = take(sizeof(float) * std::max<int64_t>(ncells, 1));
-    L.o_cnt = take(64);
     L.o_used = take(std::max<int64_t>(ncells, 1));
     L.o_bnd = take(std::max<int64_t>(ncells, 1));
     L.o_qn = take(std::max<int64_t>(ncells, 1));
@@ -344,7 +343,6 @@ DcLayout dc_layout(int64_t ncells, int64_t npts) {
     L.o_tot = take(64);
     L.o_tri = take(sizeof(int32_t) * 6 * std::max<int64_t>(npts, 1));
     L.o_hs = take(sizeof(int32_t) * hs);
-    L.o_hm = take(sizeof(int32_t) * hs);
     L.o_rep = take(sizeof(int32_t) * std::max<int64_t>(ncells, 1));
     L.o_fin = take(sizeof(int32_t) * std::max<int64_t>(ncells, 1));
     L.o_ak = take(sizeof(int64_t) * hs);
@@ -693,8 +691,8 @@ DcBatchLayout dc_batch_layout(int n, const isoext_mc_item *items, int64_t C, int
     L.o_outs = take(sizeof(iso::ItsOut) * (size_t) n);
     L.o_items = take(iso::dc_batch_item_bytes() * (size_t) n);
     L.o_citem = take(sizeof(int32_t) * c1);
-    L.o_vb = take(sizeof(int64_t) * (size_t) (n + 1));
-    L.o_qb = take(sizeof(int64_t) * (size_t) (n + 1));
+    L.o_vb = take(sizeof(int64_t) * 2 * (size_t) (n + 1));   // the two adjacent, read back together
+    L.o_qb = L.o_vb + sizeof(int64_t) * (size_t) (n + 1);
     L.o_tm = take(sizeof(uint64_t) * (size_t) std::max<int64_t>(T, 1));
     L.o_tp = take(sizeof(int32_t) * (size_t) std::max<int64_t>(T, 1));
     L.dc = dc_layout(C, 0);
@@ -808,7 +806,6 @@ int isoext_dc(const isoext_grid *g, const isoext_its *its, float reg, float svd_
     iso::DcScratch w;
     w.dual_v = dual_v ? dual_v : (float *) (ws + L.o_dual);
     w.cond = (float *) (ws + L.o_cond);
-    w.n_fp64 = (unsigned long long *) (ws + L.o_cnt);
     w.used = (uint8_t *) (ws + L.o_used);
     w.bnd = (uint8_t *) (ws + L.o_bnd);
     w.qn = (uint8_t *) (ws + L.o_qn);
@@ -816,10 +813,10 @@ int isoext_dc(const isoext_grid *g, const isoext_its *its, float reg, float svd_
     w.bsum = (int64_t *) (ws + L.o_bsum);
     w.part = (int64_t *) (ws + L.o_part);
     w.tot = (int64_t *) (ws + L.o_tot);
+    w.n_fp64 = (unsigned long long *) (w.tot + 4);
     w.tri_cells = (int32_t *) (ws + L.o_tri);
     w.cap_tri = 6 * std::max<int64_t>(its->npts, 1);
-    w.hslots = (int32_t *) (ws + L.o_hs);
-    w.slot_min = (int32_t *) (ws + L.o_hm);
+    w.hslots = (uint32_t *) (ws + L.o_hs);
     w.hmask = L.hslots - 1;
     w.akey = (int64_t *) (ws + L.o_ak);
     w.aval = (int32_t *) (ws + L.o_av);
@@ -1839,7 +1836,6 @@ int isoext_dc_batch_run(int n, const isoext_mc_item *items, const int64_t *count
     iso::DcScratch w;
     w.dual_v = (float *) (dw + D.o_dual);
     w.cond = (float *) (dw + D.o_cond);
-    w.n_fp64 = (unsigned long long *) (dw + D.o_cnt);
     w.used = (uint8_t *) (dw + D.o_used);
     w.bnd = (uint8_t *) (dw + D.o_bnd);
     w.qn = (uint8_t *) (dw + D.o_qn);
@@ -1847,10 +1843,10 @@ int isoext_dc_batch_run(int n, const isoext_mc_item *items, const int64_t *count
     w.bsum = (int64_t *) (dw + D.o_bsum);
     w.part = (int64_t *) (dw + D.o_part);
     w.tot = (int64_t *) (dw + D.o_tot);
+    w.n_fp64 = (unsigned long long *) (w.tot + 4);
     w.tri_cells = (int32_t *) (dw + D.o_tri);
     w.cap_tri = 6;
-    w.hslots = (int32_t *) (dw + D.o_hs);
-    w.slot_min = (int32_t *) (dw + D.o_hm);
+    w.hslots = (uint32_t *) (dw + D.o_hs);
     w.hmask = D.hslots - 1;
     w.akey = (int64_t *) (dw + D.o_ak);
     w.aval = (int32_t *) (dw + D.o_av);

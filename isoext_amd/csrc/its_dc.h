@@ -60,7 +60,7 @@ struct ItsIn {
 struct DcScratch {
     float *dual_v;
     float *cond;
-    unsigned long long *n_fp64;
+    unsigned long long *n_fp64;   // tot + 4
     uint8_t *used;
     uint8_t *bnd;         // vertex on its cell's box (may coincide with a neighbour's)
     uint8_t *qn;          // dense sets: quads emitted per cell
@@ -70,7 +70,7 @@ struct DcScratch {
     int64_t *tot;
     int32_t *tri_cells;
     int64_t cap_tri;
-    int32_t *hslots, *slot_min;
+    uint32_t *hslots;     // position slots of the weld
     int64_t hmask;
     int32_t *rep_slot, *final_id;
     int64_t *akey;      // active-cell hash: dense cell id -> active index
@@ -101,7 +101,7 @@ hipError_t dc_run(const GridDesc &g, const ItsIn &in, float reg, float svd_tol, 
 struct DcBatchDev {
     void *items;              // dc_batch_item_bytes() * n
     int32_t *cell_item;       // per active cell
-    int64_t *vbase, *qbase;   // n + 1 each
+    int64_t *vbase, *qbase;   // n + 1 each, qbase right after vbase
 };
 constexpr int kMaxDcBatchGrids = 256;
 // Pairs of scan scratch for nb block-sum pairs.

@@ -284,8 +284,14 @@ struct DcBatch {
     int n;
     bool tables;           // every grid has lookup tables (no active-cell hash)
     int32_t *cell_item;    // per active cell: its grid
-    int64_t *vbase;        // n + 1: first output vertex of each grid, total
+    int64_t *vbase;        // n + 1: first output vertex of each grid, total (nullptr: one grid)
     int64_t *qbase;        // n + 1: first quad of each grid, total
+};
+
+struct WeldClear {
+    uint32_t *slots;
+    int64_t hmask;
+    unsigned long long *n_fp64;
 };
 
 // ---- QEF solve ----------------------------------------------------------------
@@ -430,10 +436,10 @@ struct CsgEdges : GridEdges {
 // mass point and scaled by 1/h, one FP64-residual refinement step, FP64
 // absolute re-solve when ill-conditioned; clipped to the cell (fix_dual_v_op,
 // src/dc.cu:82-99).  Returns the condition number; on_box when the clipped
-// vertex lies on the cell's box.
+// vertex lies on the cell's box, resolved when it took the FP64 re-solve.
 template <class Ent>
 __device__ float qef_cell(const Ent &en, const float blo[3], const float bhi[3], float reg, float svd_tol,
-                          float cond_fp64, unsigned long long *n_fp64, float out[3], bool &on_box) {
+                          float cond_fp64, float out[3], bool &on_box, bool &resolved) {
     float c[3] = {0.f, 0.f, 0.f};
     for (int j = 0; j < en.n; ++j) {
         float p[3];
@@ -475,7 +481,8 @@ __device__ float qef_cell(const Ent &en, const float blo[3], const float bhi[3],
         for (int p = 0; p < 3; ++p) xs[p] += dx[p];
     }
     for (int k = 0; k < 3; ++k) out[k] = c[k] + xs[k] * h;
-    if (!(cond <= cond_fp64)) {
+    resolved = !(cond <= cond_fp64);
+    if (resolved) {
         // FP64 re-solve in absolute coordinates exactly as the reference
         // poses it (minimum-norm when singular values are truncated).
         double Ad[3][3] = {{reg, 0, 0}, {0, reg, 0}, {0, 0, reg}}, bd[3] = {0, 0, 0}, pa[3] = {0, 0, 0};
@@ -495,7 +502,6 @@ __device__ float qef_cell(const Ent &en, const float blo[3], const float bhi[3],
         double xd[3];
         pinv3<double>(Ad, bd, (double) svd_tol, xd, 12);
         for (int k = 0; k < 3; ++k) out[k] = (float) xd[k];
-        atomicAdd(n_fp64, 1ull);
     }
     on_box = false;
     for (int k = 0; k < 3; ++k) {
@@ -519,6 +525,17 @@ __device__ __forceinline__ int batch_item_of(const DcBatch &bt, const int64_t *s
     return lo_i;
 }
 
+// Flags of a cell's dual vertex (bnd).
+constexpr uint8_t kOnBox = 1, kResolved = 2;
+
+// The QEF passes clear what the weld inserts into (position slots, the
+// re-solve counter): no launch of its own.
+__device__ __forceinline__ void weld_clear(const WeldClear &c) {
+    const int64_t t = (int64_t) blockIdx.x * kBlock + threadIdx.x;
+    for (int64_t i = t; i <= c.hmask; i += (int64_t) gridDim.x * kBlock) c.slots[i] = 0xffffffffu;
+    if (t == 0) *c.n_fp64 = 0;
+}
+
 // Whether the quad of edge k of cell (x, y, z) has all four cells inside the
 // grid: across the edge, cells c - 1 and c (corner offset 0) or c and c + 1
 // (offset 1) in each of the other two axes.
@@ -532,17 +549,19 @@ __device__ __forceinline__ bool edge_interior(int k, int64_t x, int64_t y, int64
     return ok;
 }
 
-// QEF pass over an intersection set.  Also sets bnd[a] when the clipped
-// vertex lies on its cell's box (the only vertices another cell's vertex can
-// coincide with), and used[a]: with dense_used (a dense grid whose
-// intersection set is the grid's own), whether the cell belongs to a quad --
-// one of its crossing edges has all four cells around it inside the grid --
-// and qn[a], the quads the cell emits (its canonical crossing edges 0, 3, 8
-// whose lower neighbours exist); otherwise used[a] = 0, set later by the
-// quad pass.
+// QEF pass over an intersection set.  Also sets bnd[a]: kOnBox when the
+// clipped vertex lies on its cell's box (the only vertices another cell's
+// vertex can coincide with), kResolved; and with dense_used (a dense grid
+// whose intersection set is the grid's own) used[a], whether the cell belongs
+// to a quad -- one of its crossing edges has all four cells around it inside
+// the grid --, qn[a], the quads the cell emits (its canonical crossing edges
+// 0, 3, 8 whose lower neighbours exist), and qmask[a]: bit b (b = 0, 1, 2 for
+// edges 0, 3, 8) when the edge emits a quad, bit b + 3 its orientation
+// (is_out); otherwise used[a] = 0, set later by the quad pass.
 __global__ void k_dc_qef(const ItsIn in, const CellSrc s1, float reg, float svd_tol, float cond_fp64,
-                         float *dual_v, float *cond_out, unsigned long long *n_fp64, uint8_t *used, uint8_t *bnd,
-                         uint8_t *qn, bool dense_used, DcBatch bt) {
+                         float *dual_v, float *cond_out, uint8_t *used, uint8_t *bnd, uint8_t *qn, uint8_t *qmask,
+                         bool dense_used, DcBatch bt, WeldClear clr) {
+    weld_clear(clr);
     __shared__ int64_t starts[kMaxDcBatchGrids];
     if (bt.items) {
         for (int i = threadIdx.x; i < bt.n; i += kBlock) starts[i] = bt.items[i].cell0;
@@ -561,22 +580,27 @@ __global__ void k_dc_qef(const ItsIn in, const CellSrc s1, float reg, float svd_
                           grid_coord(z + 1, s.Z, s.amin[2], s.amax[2])};
     const ItsEdges en{in.points, in.normals, lo, (int) (hi - lo)};
     float out[3];
-    bool on_box;
-    const float cond = qef_cell(en, blo, bhi, reg, svd_tol, cond_fp64, n_fp64, out, on_box);
+    bool on_box, resolved;
+    const float cond = qef_cell(en, blo, bhi, reg, svd_tol, cond_fp64, out, on_box, resolved);
     for (int k = 0; k < 3; ++k) dual_v[3 * a + k] = out[k];
-    uint8_t u = 0, nq = 0;
+    uint8_t u = 0, nq = 0, qm = 0;
     if (dense_used) {
         for (int64_t j = lo; j < hi; ++j) {
             const int k = in.edge_local[j];
             const bool ok = edge_interior(k, x, y, z, s);
             u |= ok ? 1 : 0;
             // canonical edges sit at the cell's lowest corner (offsets 0): this cell emits their quad
-            nq += (ok && edge_a(k) == 0) ? 1 : 0;
+            if (ok && edge_a(k) == 0) {
+                const int b = k == 0 ? 0 : (k == 3 ? 1 : 2);
+                ++nq;
+                qm |= (uint8_t) ((in.is_out[j] ? 9u : 1u) << b);
+            }
         }
         qn[a] = nq;
+        qmask[a] = qm;
     }
     used[a] = u;
-    bnd[a] = on_box ? 1 : 0;
+    bnd[a] = (on_box ? kOnBox : 0) | (resolved ? kResolved : 0);
     if (cond_out) cond_out[a] = cond;
 }
 
@@ -590,8 +614,9 @@ __global__ void k_dc_qef(const ItsIn in, const CellSrc s1, float reg, float svd_
 // or analytic); the other variant takes the stored grids' cells.
 template <bool PROG>
 __global__ void k_dc_qef_grid(const int64_t *cell_dense, int64_t ncells, const CellSrc s1, float level, float reg,
-                              float svd_tol, float cond_fp64, float *dual_v, unsigned long long *n_fp64,
-                              uint8_t *used, uint8_t *bnd, uint8_t *qn, uint8_t *qmask, DcBatch bt) {
+                              float svd_tol, float cond_fp64, float *dual_v, uint8_t *used, uint8_t *bnd,
+                              uint8_t *qn, uint8_t *qmask, DcBatch bt, WeldClear clr) {
+    weld_clear(clr);
     __shared__ int64_t starts[kMaxDcBatchGrids];
     if (bt.items) {
         for (int i = threadIdx.x; i < bt.n; i += kBlock) starts[i] = bt.items[i].cell0;
@@ -649,16 +674,16 @@ __global__ void k_dc_qef_grid(const int64_t *cell_dense, int64_t ncells, const C
         }
     }
     float out[3];
-    bool on_box = false;
+    bool on_box = false, resolved = false;
     if (en.n > 0) {
-        if (PROG && s.csg_normals) qef_cell(en, en.lo, en.hi, reg, svd_tol, cond_fp64, n_fp64, out, on_box);
-        else qef_cell(static_cast<const GridEdges &>(en), en.lo, en.hi, reg, svd_tol, cond_fp64, n_fp64, out, on_box);
+        if (PROG && s.csg_normals) qef_cell(en, en.lo, en.hi, reg, svd_tol, cond_fp64, out, on_box, resolved);
+        else qef_cell(static_cast<const GridEdges &>(en), en.lo, en.hi, reg, svd_tol, cond_fp64, out, on_box, resolved);
     } else {
         out[0] = out[1] = out[2] = 0.0f;   // not reached: active cells have a crossing edge
     }
     for (int k = 0; k < 3; ++k) dual_v[3 * a + k] = out[k];
     used[a] = u;
-    bnd[a] = on_box ? 1 : 0;
+    bnd[a] = (on_box ? kOnBox : 0) | (resolved ? kResolved : 0);
     qn[a] = nq;
     qmask[a] = qm;
 }
@@ -781,23 +806,35 @@ __device__ __forceinline__ float dist3(const float *a, const float *b) {
     return sqrtf(s);
 }
 
-// get_triangles_op (src/dc.cu:101-157): split along the shorter diagonal.
-// Vertex id of cell a's dual vertex after the weld.
-__device__ __forceinline__ int32_t welded_id(const uint8_t *bnd, const int32_t *rep_slot, const int32_t *slot_min,
-                                             const int32_t *final_id, int32_t a) {
-    return final_id[bnd[a] ? slot_min[rep_slot[a]] : a];
-}
-
-// Quad corners go to tri_cells (cells; used[] marked here), or, when the
-// weld ran first (wd.final_id != nullptr), straight to out_f as vertex ids.
+// Vertex id of cell a's dual vertex after the weld: its own, or that of the
+// lowest cell at its position.
 struct WeldIds {
     const uint8_t *bnd;
-    const int32_t *rep_slot, *slot_min, *final_id;
+    const int32_t *rep_slot;
+    const uint32_t *slots;
+    const int32_t *final_id;
     int32_t *out_f;
 };
+__device__ __forceinline__ int32_t welded_id(const WeldIds &wd, int32_t a) {
+    return wd.final_id[(wd.bnd[a] & kOnBox) ? (int32_t) wd.slots[wd.rep_slot[a]] : a];
+}
 
+// get_triangles_op (src/dc.cu:101-157): split along the shorter diagonal.
+__device__ __forceinline__ void quad_corners(const float *dual_v, const int32_t q[4], int32_t t[6]) {
+    const bool d = dist3(dual_v + 3 * (int64_t) q[0], dual_v + 3 * (int64_t) q[2]) >
+                   dist3(dual_v + 3 * (int64_t) q[1], dual_v + 3 * (int64_t) q[3]);
+    t[0] = d ? q[1] : q[2];
+    t[1] = d ? q[3] : q[0];
+    t[2] = d ? q[0] : q[1];
+    t[3] = d ? q[3] : q[0];
+    t[4] = d ? q[1] : q[2];
+    t[5] = d ? q[2] : q[3];
+}
+
+// Sets that go through the active-cell hash: quad corners as cells, used[]
+// marked; the weld and the vertex ids come afterwards.
 __global__ void k_quad_emit(ItsIn in, CellSrc s1, ActHash ah, const int64_t *bsum_pre, const float *dual_v,
-                            int32_t *tri_cells, uint8_t *used, WeldIds wd, DcBatch bt) {
+                            int32_t *tri_cells, uint8_t *used, DcBatch bt) {
     int64_t e = (int64_t) blockIdx.x * kBlock + threadIdx.x;
     int64_t nq = 0;
     int64_t q[4] = {0, 0, 0, 0};
@@ -818,19 +855,9 @@ __global__ void k_quad_emit(ItsIn in, CellSrc s1, ActHash ah, const int64_t *bsu
     // batch: the grid's first entry records the grid's first quad
     if (bt.items && e < in.npts && e == in.cell_offsets[bt.items[item].cell0]) bt.qbase[item] = slot;
     if (!nq) return;
-    const float *v0 = dual_v + 3 * q[0], *v1 = dual_v + 3 * q[1], *v2 = dual_v + 3 * q[2], *v3 = dual_v + 3 * q[3];
+    const int32_t c[4] = {(int32_t) q[0], (int32_t) q[1], (int32_t) q[2], (int32_t) q[3]};
     int32_t t[6];
-    if (dist3(v0, v2) > dist3(v1, v3)) {
-        int32_t u[6] = {(int32_t) q[1], (int32_t) q[3], (int32_t) q[0], (int32_t) q[3], (int32_t) q[1], (int32_t) q[2]};
-        for (int k = 0; k < 6; ++k) t[k] = u[k];
-    } else {
-        int32_t u[6] = {(int32_t) q[2], (int32_t) q[0], (int32_t) q[1], (int32_t) q[0], (int32_t) q[2], (int32_t) q[3]};
-        for (int k = 0; k < 6; ++k) t[k] = u[k];
-    }
-    if (wd.final_id) {
-        for (int k = 0; k < 6; ++k) wd.out_f[6 * slot + k] = welded_id(wd.bnd, wd.rep_slot, wd.slot_min, wd.final_id, t[k]);
-        return;
-    }
+    quad_corners(dual_v, c, t);
     for (int k = 0; k < 6; ++k) tri_cells[6 * slot + k] = t[k];
     for (int k = 0; k < 4; ++k) used[q[k]] = 1;
 }
@@ -842,52 +869,79 @@ __global__ void k_quad_emit(ItsIn in, CellSrc s1, ActHash ah, const int64_t *bsu
 // only those go through the position hash; every other used vertex is its
 // own representative.
 
-__global__ void k_pos_insert(const float *dv, const uint8_t *used, const uint8_t *bnd, int64_t n, int32_t *slots,
+// A slot holds the lowest cell at its position (all ones: empty): whichever
+// cell of a position arrives first claims the slot, the others lower it.
+__global__ void k_pos_insert(const float *dv, const uint8_t *used, const uint8_t *bnd, int64_t n, uint32_t *slots,
                              int64_t mask, int32_t *rep, const int32_t *cell_item) {
     int64_t a = (int64_t) blockIdx.x * kBlock + threadIdx.x;
-    if (a >= n || !used[a] || !bnd[a]) return;
+    if (a >= n || !used[a] || !(bnd[a] & kOnBox)) return;
     float x = dv[3 * a], y = dv[3 * a + 1], z = dv[3 * a + 2];
     // batches: vertices of different grids never weld (the grid joins the hash and the test)
     const int32_t item = cell_item ? cell_item[a] : 0;
     uint64_t h = (f3_hash(x, y, z) ^ (uint64_t) mix64((uint64_t) item)) & (uint64_t) mask;
     for (int64_t probe = 0; probe <= mask; ++probe) {
         int64_t sl = (int64_t) ((h + probe) & (uint64_t) mask);
-        int32_t cur = slots[sl];
-        if (cur < 0) {
-            int32_t prev = atomicCAS(&slots[sl], -1, (int32_t) a);
-            if (prev < 0) {
+        uint32_t cur = slots[sl];
+        if (cur == 0xffffffffu) {
+            cur = atomicCAS(&slots[sl], 0xffffffffu, (uint32_t) a);
+            if (cur == 0xffffffffu) {
                 rep[a] = (int32_t) sl;
                 return;
             }
-            cur = prev;
         }
-        if (dv[3 * cur] == x && dv[3 * cur + 1] == y && dv[3 * cur + 2] == z &&
+        // any cell the slot has held is at the slot's position
+        if (dv[3 * (int64_t) cur] == x && dv[3 * (int64_t) cur + 1] == y && dv[3 * (int64_t) cur + 2] == z &&
             (!cell_item || cell_item[cur] == item)) {
+            atomicMin(&slots[sl], (uint32_t) a);
             rep[a] = (int32_t) sl;
             return;
         }
     }
 }
 
-__global__ void k_slot_min(const uint8_t *used, const uint8_t *bnd, int64_t n, const int32_t *rep_slot,
-                           int32_t *slot_min) {
-    int64_t a = (int64_t) blockIdx.x * kBlock + threadIdx.x;
-    if (a >= n || !used[a] || !bnd[a]) return;
-    atomicMin(&slot_min[rep_slot[a]], (int32_t) a);
-}
-
 // Used vertex a is kept when it represents its position.
 __device__ __forceinline__ bool kept_vertex(const uint8_t *used, const uint8_t *bnd, const int32_t *rep_slot,
-                                            const int32_t *slot_min, int64_t a) {
-    return used[a] && (!bnd[a] || slot_min[rep_slot[a]] == (int32_t) a);
+                                            const uint32_t *slots, int64_t a) {
+    return used[a] && (!(bnd[a] & kOnBox) || slots[rep_slot[a]] == (uint32_t) a);
+}
+
+// (kept vertices, quads) of the blocks before this one: from the scan, or,
+// with at most kDirectBlocks blocks (262 k cells), summed here from the block
+// sums by every workgroup (a few KB from the L2) instead of a scan launch
+// between; the last block then leaves the totals.  The scan took 4 us and its
+// launch gap 2, the sums add under 1 us to each of the two kernels that read
+// them; past some thousand blocks the reads grow past that.  kBlock threads.
+constexpr int64_t kDirectBlocks = 1024;
+__device__ __forceinline__ void block_base(const int64_t *bsum, bool scanned, int64_t *tot, int64_t &bv, int64_t &bq) {
+    const int64_t blk = blockIdx.x;
+    if (scanned) {
+        bv = bsum[2 * blk];
+        bq = bsum[2 * blk + 1];
+        return;
+    }
+    int64_t v = 0, q = 0;
+#pragma unroll 4
+    for (int64_t i = threadIdx.x; i < blk; i += kBlock) {
+        v += bsum[2 * i];
+        q += bsum[2 * i + 1];
+    }
+    int64_t ev, eq;
+    block_scan2(v, q, ev, eq, bv, bq);
+    if (tot && threadIdx.x == 0 && blk == (int64_t) gridDim.x - 1) {
+        tot[0] = bv + bsum[2 * blk];
+        tot[1] = bq + bsum[2 * blk + 1];
+    }
 }
 
 // Block sums of (kept vertices, quads per cell from qn, or 0 without it).
+// The FP64 re-solves are counted on the way.
 __global__ void k_keep_flags(const uint8_t *used, const uint8_t *bnd, int64_t n, const int32_t *rep_slot,
-                             const int32_t *slot_min, const uint8_t *qn, int64_t *bsum) {
+                             const uint32_t *slots, const uint8_t *qn, int64_t *bsum, unsigned long long *n_fp64) {
     int64_t a = (int64_t) blockIdx.x * kBlock + threadIdx.x;
-    int64_t k = (a < n && kept_vertex(used, bnd, rep_slot, slot_min, a)) ? 1 : 0;
+    int64_t k = (a < n && kept_vertex(used, bnd, rep_slot, slots, a)) ? 1 : 0;
     int64_t q = (qn && a < n) ? qn[a] : 0;
+    const uint64_t res = __ballot(a < n && (bnd[a] & kResolved));
+    if (res && (threadIdx.x & 63) == 0) atomicAdd(n_fp64, (unsigned long long) __popcll(res));
     int64_t ek, eq, tk, tq;
     block_scan2(k, q, ek, eq, tk, tq);
     if (threadIdx.x == 0) {
@@ -896,17 +950,20 @@ __global__ void k_keep_flags(const uint8_t *used, const uint8_t *bnd, int64_t n,
     }
 }
 
+// tot (optional): the totals, left by the last block where the sums are not
+// scanned.
 __global__ void k_keep_emit(const float *dv, const uint8_t *used, const uint8_t *bnd, int64_t n,
-                            const int32_t *rep_slot, const int32_t *slot_min, const int64_t *bsum_pre,
-                            int32_t *final_id, float *out_v, int32_t *out_vcell, DcBatch bt) {
+                            const int32_t *rep_slot, const uint32_t *slots, const int64_t *bsum, bool scanned,
+                            int64_t *tot, int32_t *final_id, float *out_v, int32_t *out_vcell, DcBatch bt) {
     int64_t a = (int64_t) blockIdx.x * kBlock + threadIdx.x;
-    int64_t k = (a < n && kept_vertex(used, bnd, rep_slot, slot_min, a)) ? 1 : 0;
-    int64_t ek, d, tk, td;
+    int64_t k = (a < n && kept_vertex(used, bnd, rep_slot, slots, a)) ? 1 : 0;
+    int64_t ek, d, tk, td, bv, bq;
+    block_base(bsum, scanned, tot, bv, bq);
     block_scan2(k, 0, ek, d, tk, td);
     if (!k) return;
-    const int64_t id = bsum_pre[2 * blockIdx.x] + ek;
+    const int64_t id = bv + ek;
     // batch: face corners use grid-local vertex ids
-    final_id[a] = (int32_t) (bt.items ? id - bt.vbase[bt.cell_item[a]] : id);
+    final_id[a] = (int32_t) (bt.vbase ? id - bt.vbase[bt.cell_item[a]] : id);
     out_v[3 * id + 0] = dv[3 * a + 0];
     out_v[3 * id + 1] = dv[3 * a + 1];
     out_v[3 * id + 2] = dv[3 * a + 2];
@@ -914,12 +971,10 @@ __global__ void k_keep_emit(const float *dv, const uint8_t *used, const uint8_t 
 }
 
 // Face corners: 6 per quad; the quad count is read from the device.
-__global__ void k_remap_faces(const int32_t *tri_cells, const int64_t *nquads, const uint8_t *bnd,
-                              const int32_t *rep_slot, const int32_t *slot_min, const int32_t *final_id,
-                              int32_t *out_f) {
+__global__ void k_remap_faces(const int32_t *tri_cells, const int64_t *nquads, WeldIds wd) {
     int64_t i = (int64_t) blockIdx.x * kBlock + threadIdx.x;
     if (i >= 6 * *nquads) return;
-    out_f[i] = welded_id(bnd, rep_slot, slot_min, final_id, tri_cells[i]);
+    wd.out_f[i] = welded_id(wd, tri_cells[i]);
 }
 
 // Batch: first output vertex of each grid = kept vertices before its first
@@ -928,7 +983,7 @@ __global__ void k_remap_faces(const int32_t *tri_cells, const int64_t *nquads, c
 // With qn (quads counted per cell), the first quads too: bsum_pre's second
 // component and tot[3] hold the quad scan.
 __global__ void k_item_vbase(DcBatch bt, const uint8_t *used, const uint8_t *bnd, const int32_t *rep_slot,
-                             const int32_t *slot_min, const uint8_t *qn, const int64_t *bsum_pre, int64_t ncells,
+                             const uint32_t *slots, const uint8_t *qn, const int64_t *bsum_pre, int64_t ncells,
                              const int64_t *tot) {
     __shared__ int part[kBlock / 64], partq[kBlock / 64];
     const int i = blockIdx.x;
@@ -945,7 +1000,7 @@ __global__ void k_item_vbase(DcBatch bt, const uint8_t *used, const uint8_t *bnd
         return;
     }
     const int64_t blk = c0 / kBlock, a = blk * kBlock + threadIdx.x;
-    int k = (a < c0 && kept_vertex(used, bnd, rep_slot, slot_min, a)) ? 1 : 0;
+    int k = (a < c0 && kept_vertex(used, bnd, rep_slot, slots, a)) ? 1 : 0;
     int q = (qn && a < c0) ? qn[a] : 0;
     for (int o = 32; o > 0; o >>= 1) {
         k += __shfl_down(k, o);
@@ -967,108 +1022,67 @@ __global__ void k_item_vbase(DcBatch bt, const uint8_t *used, const uint8_t *bnd
     }
 }
 
-// Quads of dense sets, one thread per active cell: the cell's canonical
-// entries in entry order (the per-entry kernel's order), at the cell's
-// offset in the quad scan (second component of bsum_pre); corners are
-// written as welded vertex ids.
-__global__ void k_quad_emit_cells(ItsIn in, CellSrc s1, const uint8_t *qn, const int64_t *bsum_pre,
-                                  const float *dual_v, WeldIds wd, DcBatch bt) {
-    const int64_t a = (int64_t) blockIdx.x * kBlock + threadIdx.x;
-    const int64_t nq = a < in.ncells ? qn[a] : 0;
-    int64_t ed, eq, td, tq;
-    block_scan2(0, nq, ed, eq, td, tq);
-    if (!nq) return;
-    int64_t slot = bsum_pre[2 * blockIdx.x + 1] + eq;
-    const DcItem *it = nullptr;
-    DcItem one;
-    if (bt.items) {
-        it = &bt.items[bt.cell_item[a]];
-    } else {
-        one = DcItem{s1, 0, 0, in.amask_tab, in.apre_tab, (s1.Z + 63) / 64, 0.0f};
-        it = &one;
+// Quads of a dense grid, one thread per active cell: its canonical edges from
+// qmask in edge order (0, 3, 8: the entry order of the intersection set),
+// neighbours from the lookup tables, the reference's orientation and
+// shorter-diagonal split, corners as welded vertex ids at the cell's offset in
+// the quad scan.  A chain of dependent loads (table, vertices, ids) for each
+// quad: the edges are unrolled with constant neighbour offsets, so that
+// nothing is indexed in scratch and the four corners' loads overlap (52 k
+// cells: 14 -> 9.7 us; the 207 k cells of a 256^3 set: 34 -> 14 us).
+template <int B>
+__device__ __forceinline__ void grid_quad(const CellSrc &s, const uint64_t *amask, const int32_t *apre, int64_t W,
+                                          int64_t a, int64_t x, int64_t y, int64_t z, int qm, const float *dual_v,
+                                          const WeldIds &wd, int64_t slot) {
+    // edge_neighbors_table (src/shared_luts.cu:78-82) of edges 0 (along z), 3 (y), 8 (x)
+    constexpr int off[3][3][3] = {{{1, 0, 0}, {1, 1, 0}, {0, 1, 0}},
+                                  {{0, 0, 1}, {1, 0, 1}, {1, 0, 0}},
+                                  {{0, 1, 0}, {0, 1, 1}, {0, 0, 1}}};
+    int32_t c[4];
+    c[0] = (int32_t) a;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        const int64_t cz = z - off[B][j][2], t = ((x - off[B][j][0]) * (s.Y - 1) + (y - off[B][j][1])) * W + (cz >> 6);
+        c[j + 1] = apre[t] + __popcll(amask[t] & ((1ull << (cz & 63)) - 1ull));
     }
-    const ActHash ah{nullptr, nullptr, 0};
-    const int64_t lo = in.cell_offsets[a], hi = in.cell_offsets[a + 1];
-    for (int64_t e = lo; e < hi; ++e) {
-        int64_t q[4];
-        if (!entry_quad(in, it->s, ah, e, q, true, it->key_base, it)) continue;
-        const float *v0 = dual_v + 3 * q[0], *v1 = dual_v + 3 * q[1], *v2 = dual_v + 3 * q[2],
-                    *v3 = dual_v + 3 * q[3];
-        int32_t t[6];
-        if (dist3(v0, v2) > dist3(v1, v3)) {
-            const int32_t u[6] = {(int32_t) q[1], (int32_t) q[3], (int32_t) q[0],
-                                  (int32_t) q[3], (int32_t) q[1], (int32_t) q[2]};
-            for (int k = 0; k < 6; ++k) t[k] = u[k];
-        } else {
-            const int32_t u[6] = {(int32_t) q[2], (int32_t) q[0], (int32_t) q[1],
-                                  (int32_t) q[0], (int32_t) q[2], (int32_t) q[3]};
-            for (int k = 0; k < 6; ++k) t[k] = u[k];
-        }
-        for (int k = 0; k < 6; ++k)
-            wd.out_f[6 * slot + k] = welded_id(wd.bnd, wd.rep_slot, wd.slot_min, wd.final_id, t[k]);
-        ++slot;
-    }
+    const bool out = (qm >> (B + 3)) & 1;
+    const int32_t q[4] = {out ? c[0] : c[3], out ? c[1] : c[2], out ? c[2] : c[1], out ? c[3] : c[0]};
+    int32_t t[6], id[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) id[k] = welded_id(wd, q[k]);
+    const bool d = dist3(dual_v + 3 * (int64_t) q[0], dual_v + 3 * (int64_t) q[2]) >
+                   dist3(dual_v + 3 * (int64_t) q[1], dual_v + 3 * (int64_t) q[3]);
+    t[0] = d ? id[1] : id[2];
+    t[1] = d ? id[3] : id[0];
+    t[2] = d ? id[0] : id[1];
+    t[3] = d ? id[3] : id[0];
+    t[4] = d ? id[1] : id[2];
+    t[5] = d ? id[2] : id[3];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) wd.out_f[6 * slot + k] = t[k];
 }
 
-// Quads of a dense grid without an intersection set, one thread per active
-// cell: its canonical edges from qmask in edge order (0, 3, 8: the entry
-// order of the intersection set), neighbours from the lookup tables, the
-// reference's orientation and shorter-diagonal split, corners as welded
-// vertex ids at the cell's offset in the quad scan.
 __global__ void k_quad_emit_grid(const int64_t *cell_dense, int64_t ncells, CellSrc s1, const uint64_t *amask_tab,
                                  const int32_t *apre_tab, const uint8_t *qn, const uint8_t *qmask,
-                                 const int64_t *bsum_pre, const float *dual_v, WeldIds wd, DcBatch bt) {
+                                 const int64_t *bsum, bool scanned, const float *dual_v, WeldIds wd, DcBatch bt) {
     const int64_t a = (int64_t) blockIdx.x * kBlock + threadIdx.x;
     const int64_t nq = a < ncells ? qn[a] : 0;
-    int64_t ed, eq, td, tq;
+    int64_t ed, eq, td, tq, bv, bq;
+    block_base(bsum, scanned, nullptr, bv, bq);
     block_scan2(0, nq, ed, eq, td, tq);
     if (!nq) return;
-    int64_t slot = bsum_pre[2 * blockIdx.x + 1] + eq;
-    DcItem one;
-    const DcItem *it;
-    if (bt.items) {
-        it = &bt.items[bt.cell_item[a]];
-    } else {
-        one = DcItem{s1, 0, 0, amask_tab, apre_tab, (s1.Z + 63) / 64, 0.0f};
-        it = &one;
-    }
+    int64_t slot = bq + eq;
+    const DcItem *it = bt.items ? &bt.items[bt.cell_item[a]] : nullptr;
+    const CellSrc &s = it ? it->s : s1;
+    const uint64_t *am = it ? it->amask : amask_tab;
+    const int32_t *ap = it ? it->apre : apre_tab;
+    const int64_t W = it ? it->W : (s1.Z + 63) / 64;
     int64_t x, y, z;
-    cell_xyz(it->s, cell_dense[a], x, y, z);
+    cell_xyz(s, cell_dense[a], x, y, z);
     const int qm = qmask[a];
-    for (int b = 0; b < 3; ++b) {
-        if (!((qm >> b) & 1)) continue;
-        const int axis = edge_axis(b == 0 ? 0 : (b == 1 ? 3 : 8));
-        int64_t q[4];
-        q[0] = a;
-        for (int j = 1; j < 4; ++j)
-            q[j] = active_of_tab(*it, x - kNb[axis][j][0], y - kNb[axis][j][1], z - kNb[axis][j][2]);
-        if (!((qm >> (b + 3)) & 1)) {
-            const int64_t t0 = q[0], t1 = q[1];
-            q[0] = q[3];
-            q[1] = q[2];
-            q[2] = t1;
-            q[3] = t0;
-        }
-        const float *v0 = dual_v + 3 * q[0], *v1 = dual_v + 3 * q[1], *v2 = dual_v + 3 * q[2],
-                    *v3 = dual_v + 3 * q[3];
-        int32_t t[6];
-        if (dist3(v0, v2) > dist3(v1, v3)) {
-            const int32_t u[6] = {(int32_t) q[1], (int32_t) q[3], (int32_t) q[0],
-                                  (int32_t) q[3], (int32_t) q[1], (int32_t) q[2]};
-            for (int k = 0; k < 6; ++k) t[k] = u[k];
-        } else {
-            const int32_t u[6] = {(int32_t) q[2], (int32_t) q[0], (int32_t) q[1],
-                                  (int32_t) q[0], (int32_t) q[2], (int32_t) q[3]};
-            for (int k = 0; k < 6; ++k) t[k] = u[k];
-        }
-        for (int k = 0; k < 6; ++k)
-            wd.out_f[6 * slot + k] = welded_id(wd.bnd, wd.rep_slot, wd.slot_min, wd.final_id, t[k]);
-        ++slot;
-    }
-}
-
-__global__ void k_copy_i64(int64_t *dst, const int64_t *src) {
-    if (threadIdx.x == 0) *dst = *src;
+    if (qm & 1) grid_quad<0>(s, am, ap, W, a, x, y, z, qm, dual_v, wd, slot++);
+    if (qm & 2) grid_quad<1>(s, am, ap, W, a, x, y, z, qm, dual_v, wd, slot++);
+    if (qm & 4) grid_quad<2>(s, am, ap, W, a, x, y, z, qm, dual_v, wd, slot++);
 }
 
 // First quads of grids without cells (no thread recorded them: they equal
@@ -1083,16 +1097,9 @@ __global__ void k_item_qbase(DcBatch bt, int64_t ncells, const int64_t *tot) {
     }
 }
 
-__global__ void k_fill_i32(int32_t *p, int64_t n, int32_t v) {
-    for (int64_t i = (int64_t) blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t) gridDim.x * kBlock) p[i] = v;
-}
 __global__ void k_fill_i64(int64_t *p, int64_t n, int64_t v) {
     for (int64_t i = (int64_t) blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t) gridDim.x * kBlock) p[i] = v;
 }
-__global__ void k_fill_u8(uint8_t *p, int64_t n, uint8_t v) {
-    for (int64_t i = (int64_t) blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t) gridDim.x * kBlock) p[i] = v;
-}
-
 // exclusive scan of block sums (pairs), single block, in place; totals out
 // Parallel exclusive scan of the block-sum pairs for large inputs: chunk
 // sums, one workgroup over the chunk sums, then each chunk rescanned with its
@@ -1379,6 +1386,33 @@ static void scan_pairs(int64_t *bsum, int64_t nb, int64_t *tot, int64_t *part, h
                        (const int64_t *) part);
 }
 
+// Weld, vertex and quad offsets, vertices, faces.  Leaves the totals in
+// w.tot[2] (vertices) and, with tables (dense grids), w.tot[3] (quads).
+static void weld_and_emit(const CellSrc &s, const ItsIn &in, const uint64_t *amask, const int32_t *apre, bool tables,
+                          DcScratch &w, const DcBatch &bt, hipStream_t st) {
+    const unsigned nbv = nblocks(in.ncells);
+    const WeldIds wd{w.bnd, w.rep_slot, w.hslots, w.final_id, w.out_f};
+    const uint8_t *qn = tables ? w.qn : nullptr;
+    hipLaunchKernelGGL(k_pos_insert, dim3(nbv), dim3(kBlock), 0, st, w.dual_v, w.used, w.bnd, in.ncells, w.hslots,
+                       w.hmask, w.rep_slot, (const int32_t *) bt.cell_item);
+    hipLaunchKernelGGL(k_keep_flags, dim3(nbv), dim3(kBlock), 0, st, w.used, w.bnd, in.ncells, w.rep_slot, w.hslots,
+                       qn, w.bsum, w.n_fp64);
+    // several grids need the offsets of their first cells: scanned apart
+    const bool scanned = bt.vbase || nbv > kDirectBlocks;
+    if (scanned) scan_pairs(w.bsum, (int64_t) nbv, w.tot + 2, w.part, st);
+    if (bt.vbase)
+        hipLaunchKernelGGL(k_item_vbase, dim3(bt.n), dim3(kBlock), 0, st, bt, w.used, w.bnd, w.rep_slot, w.hslots, qn,
+                           w.bsum, in.ncells, (const int64_t *) w.tot);
+    hipLaunchKernelGGL(k_keep_emit, dim3(nbv), dim3(kBlock), 0, st, w.dual_v, w.used, w.bnd, in.ncells, w.rep_slot,
+                       w.hslots, (const int64_t *) w.bsum, scanned, w.tot + 2, w.final_id, w.out_v, w.out_vcell, bt);
+    if (tables)
+        hipLaunchKernelGGL(k_quad_emit_grid, dim3(nbv), dim3(kBlock), 0, st, in.cell_dense, in.ncells, s, amask, apre,
+                           (const uint8_t *) w.qn, (const uint8_t *) w.qmask, (const int64_t *) w.bsum, scanned,
+                           w.dual_v, wd, bt);
+    else
+        hipLaunchKernelGGL(k_remap_faces, dim3(nblocks(6 * in.npts)), dim3(kBlock), 0, st, w.tri_cells, w.tot, wd);
+}
+
 static hipError_t dc_launch(const CellSrc &s, const ItsIn &in, float reg, float svd_tol, float cond_fp64,
                             DcScratch &w, const DcBatch &bt, hipStream_t st) {
     // Dense grids with lookup tables (the intersection set is the grid's
@@ -1388,11 +1422,11 @@ static hipError_t dc_launch(const CellSrc &s, const ItsIn &in, float reg, float 
     // scan.  Otherwise: hash, per-entry quads (marking used[]), weld, face
     // remap.
     const bool tables = bt.items ? bt.tables : (in.amask_tab && in.apre_tab && !s.ids);
-    hipLaunchKernelGGL(k_fill_i64, dim3(1), dim3(64), 0, st, (int64_t *) w.n_fp64, (int64_t) 1, (int64_t) 0);
+    const WeldClear clr{w.hslots, w.hmask, w.n_fp64};
     hipLaunchKernelGGL(k_dc_qef, dim3(nblocks(in.ncells)), dim3(kBlock), 0, st, in, s, reg, svd_tol, cond_fp64,
-                       w.dual_v, w.cond, w.n_fp64, w.used, w.bnd, w.qn, tables, bt);
+                       w.dual_v, w.cond, w.used, w.bnd, w.qn, w.qmask, tables, bt, clr);
     const ActHash ah{w.akey, w.aval, w.amask};
-    const unsigned nbq = nblocks(in.npts), nbv = nblocks(in.ncells);
+    const unsigned nbq = nblocks(in.npts);
     if (!tables) {   // active-cell hash for the quads' neighbour lookups, then the quads
         const unsigned nbh = (unsigned) std::min<int64_t>(nblocks(w.amask + 1), 4096);
         hipLaunchKernelGGL(k_fill_i64, dim3(nbh), dim3(kBlock), 0, st, w.akey, w.amask + 1, (int64_t) -1);
@@ -1401,34 +1435,10 @@ static hipError_t dc_launch(const CellSrc &s, const ItsIn &in, float reg, float 
         hipLaunchKernelGGL(k_quad_count, dim3(nbq), dim3(kBlock), 0, st, in, s, ah, w.bsum, bt);
         scan_pairs(w.bsum, (int64_t) nbq, w.tot, w.part, st);
         hipLaunchKernelGGL(k_quad_emit, dim3(nbq), dim3(kBlock), 0, st, in, s, ah, w.bsum, w.dual_v, w.tri_cells,
-                           w.used, WeldIds{}, bt);
+                           w.used, bt);
         if (bt.items) hipLaunchKernelGGL(k_item_qbase, dim3(1), dim3(64), 0, st, bt, in.ncells, (const int64_t *) w.tot);
     }
-    // weld dual vertices by position
-    hipLaunchKernelGGL(k_fill_i32, dim3(nblocks(w.hmask + 1)), dim3(kBlock), 0, st, w.hslots, w.hmask + 1, -1);
-    hipLaunchKernelGGL(k_fill_i32, dim3(nblocks(w.hmask + 1)), dim3(kBlock), 0, st, w.slot_min, w.hmask + 1,
-                       INT32_MAX);
-    hipLaunchKernelGGL(k_pos_insert, dim3(nblocks(in.ncells)), dim3(kBlock), 0, st, w.dual_v, w.used, w.bnd,
-                       in.ncells, w.hslots, w.hmask, w.rep_slot, (const int32_t *) bt.cell_item);
-    hipLaunchKernelGGL(k_slot_min, dim3(nblocks(in.ncells)), dim3(kBlock), 0, st, w.used, w.bnd, in.ncells,
-                       w.rep_slot, w.slot_min);
-    const uint8_t *qn = tables ? w.qn : nullptr;
-    hipLaunchKernelGGL(k_keep_flags, dim3(nbv), dim3(kBlock), 0, st, w.used, w.bnd, in.ncells, w.rep_slot,
-                       w.slot_min, qn, w.bsum);
-    // tot[2] = kept vertices, tot[3] = quads (tables); tot[0] = quads after the copy
-    scan_pairs(w.bsum, (int64_t) nbv, w.tot + 2, w.part, st);
-    if (tables) hipLaunchKernelGGL(k_copy_i64, dim3(1), dim3(64), 0, st, w.tot, (const int64_t *) (w.tot + 3));
-    if (bt.items)
-        hipLaunchKernelGGL(k_item_vbase, dim3(bt.n), dim3(kBlock), 0, st, bt, w.used, w.bnd, w.rep_slot, w.slot_min,
-                           qn, w.bsum, in.ncells, (const int64_t *) w.tot);
-    hipLaunchKernelGGL(k_keep_emit, dim3(nbv), dim3(kBlock), 0, st, w.dual_v, w.used, w.bnd, in.ncells,
-                       w.rep_slot, w.slot_min, w.bsum, w.final_id, w.out_v, w.out_vcell, bt);
-    if (tables)
-        hipLaunchKernelGGL(k_quad_emit_cells, dim3(nbv), dim3(kBlock), 0, st, in, s, w.qn, w.bsum, w.dual_v,
-                           WeldIds{w.bnd, w.rep_slot, w.slot_min, w.final_id, w.out_f}, bt);
-    else
-        hipLaunchKernelGGL(k_remap_faces, dim3(nblocks(6 * in.npts)), dim3(kBlock), 0, st, w.tri_cells, w.tot,
-                           w.bnd, w.rep_slot, w.slot_min, w.final_id, w.out_f);
+    weld_and_emit(s, in, in.amask_tab, in.apre_tab, tables, w, bt, st);
     return hipGetLastError();
 }
 
@@ -1440,32 +1450,17 @@ static hipError_t dc_launch_grid(const CellSrc &s, const int64_t *cell_dense, in
                                  DcScratch &w, const DcBatch &bt, hipStream_t st, bool has_grid = true,
                                  bool has_prog = false) {
     const unsigned nbv = nblocks(ncells);
-    hipLaunchKernelGGL(k_fill_i64, dim3(1), dim3(64), 0, st, (int64_t *) w.n_fp64, (int64_t) 1, (int64_t) 0);
+    const WeldClear clr{w.hslots, w.hmask, w.n_fp64};
     if (has_grid)
         hipLaunchKernelGGL(k_dc_qef_grid<false>, dim3(nbv), dim3(kBlock), 0, st, cell_dense, ncells, s, level, reg,
-                           svd_tol, cond_fp64, w.dual_v, w.n_fp64, w.used, w.bnd, w.qn, w.qmask, bt);
+                           svd_tol, cond_fp64, w.dual_v, w.used, w.bnd, w.qn, w.qmask, bt, clr);
     if (has_prog)
         hipLaunchKernelGGL(k_dc_qef_grid<true>, dim3(nbv), dim3(kBlock), 0, st, cell_dense, ncells, s, level, reg,
-                           svd_tol, cond_fp64, w.dual_v, w.n_fp64, w.used, w.bnd, w.qn, w.qmask, bt);
-    hipLaunchKernelGGL(k_fill_i32, dim3(nblocks(w.hmask + 1)), dim3(kBlock), 0, st, w.hslots, w.hmask + 1, -1);
-    hipLaunchKernelGGL(k_fill_i32, dim3(nblocks(w.hmask + 1)), dim3(kBlock), 0, st, w.slot_min, w.hmask + 1,
-                       INT32_MAX);
-    hipLaunchKernelGGL(k_pos_insert, dim3(nbv), dim3(kBlock), 0, st, w.dual_v, w.used, w.bnd, ncells, w.hslots,
-                       w.hmask, w.rep_slot, (const int32_t *) bt.cell_item);
-    hipLaunchKernelGGL(k_slot_min, dim3(nbv), dim3(kBlock), 0, st, w.used, w.bnd, ncells, w.rep_slot, w.slot_min);
-    hipLaunchKernelGGL(k_keep_flags, dim3(nbv), dim3(kBlock), 0, st, w.used, w.bnd, ncells, w.rep_slot, w.slot_min,
-                       (const uint8_t *) w.qn, w.bsum);
-    // tot[2] = kept vertices, tot[3] = quads; tot[0] = quads after the copy
-    scan_pairs(w.bsum, (int64_t) nbv, w.tot + 2, w.part, st);
-    hipLaunchKernelGGL(k_copy_i64, dim3(1), dim3(64), 0, st, w.tot, (const int64_t *) (w.tot + 3));
-    if (bt.items)
-        hipLaunchKernelGGL(k_item_vbase, dim3(bt.n), dim3(kBlock), 0, st, bt, w.used, w.bnd, w.rep_slot, w.slot_min,
-                           (const uint8_t *) w.qn, w.bsum, ncells, (const int64_t *) w.tot);
-    hipLaunchKernelGGL(k_keep_emit, dim3(nbv), dim3(kBlock), 0, st, w.dual_v, w.used, w.bnd, ncells, w.rep_slot,
-                       w.slot_min, w.bsum, w.final_id, w.out_v, w.out_vcell, bt);
-    hipLaunchKernelGGL(k_quad_emit_grid, dim3(nbv), dim3(kBlock), 0, st, cell_dense, ncells, s, amask, apre,
-                       (const uint8_t *) w.qn, (const uint8_t *) w.qmask, w.bsum, w.dual_v,
-                       WeldIds{w.bnd, w.rep_slot, w.slot_min, w.final_id, w.out_f}, bt);
+                           svd_tol, cond_fp64, w.dual_v, w.used, w.bnd, w.qn, w.qmask, bt, clr);
+    ItsIn in{};
+    in.ncells = ncells;
+    in.cell_dense = cell_dense;
+    weld_and_emit(s, in, amask, apre, true, w, bt, st);
     return hipGetLastError();
 }
 
@@ -1485,10 +1480,9 @@ hipError_t dc_run(const GridDesc &g, const ItsIn &in, float reg, float svd_tol, 
     };
     thread_local PinnedTot pt;
     if (!pt.p) ISO_TRY(hipHostMalloc((void **) &pt.p, 8 * sizeof(int64_t), 0));
-    ISO_TRY(hipMemcpyAsync(pt.p, w.tot, 4 * sizeof(int64_t), hipMemcpyDeviceToHost, st));
-    ISO_TRY(hipMemcpyAsync(pt.p + 4, w.n_fp64, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+    ISO_TRY(hipMemcpyAsync(pt.p, w.tot, 5 * sizeof(int64_t), hipMemcpyDeviceToHost, st));   // n_fp64 is tot[4]
     ISO_TRY(hipStreamSynchronize(st));
-    const int64_t nq = pt.p[0];
+    const int64_t nq = in.amask_tab && in.apre_tab && !s.ids ? pt.p[3] : pt.p[0];
     w.nquads = nq;
     nv = pt.p[2];
     nf = 2 * nq;
@@ -1515,7 +1509,7 @@ hipError_t dc_run_batch(int n, const GridDesc *g, const int64_t *cell0, const ui
         }
     };
     thread_local PinnedStage ps;
-    const size_t up = sizeof(DcItem) * (size_t) n, down = sizeof(int64_t) * (2 * (size_t) n + 3);
+    const size_t up = sizeof(DcItem) * (size_t) n, down = sizeof(int64_t) * (2 * (size_t) n + 7);
     const size_t want = ((up + 255) & ~size_t(255)) + down;
     if (ps.bytes < want) {
         if (ps.p) ISO_TRY(hipHostFree(ps.p));
@@ -1544,22 +1538,25 @@ hipError_t dc_run_batch(int n, const GridDesc *g, const int64_t *cell0, const ui
     if (levels && !tables) return hipErrorInvalidValue;   // the grid path needs the tables
     int64_t *rb = (int64_t *) (ps.p + ((up + 255) & ~size_t(255)));
     ISO_TRY(hipMemcpyAsync(d.items, hi, up, hipMemcpyHostToDevice, st));
-    const DcBatch bt{(const DcItem *) d.items, n, tables, d.cell_item, d.vbase, d.qbase};
+    // one grid starts at vertex 0 and quad 0
+    const DcBatch bt{(const DcItem *) d.items, n, tables, d.cell_item, n > 1 ? d.vbase : nullptr, d.qbase};
     if (levels)
         ISO_TRY(dc_launch_grid(hi[0].s, in.cell_dense, in.ncells, nullptr, nullptr, 0.0f, reg, svd_tol, cond_fp64, w,
                                bt, st, has_grid, has_prog));
     else
         ISO_TRY(dc_launch(hi[0].s, in, reg, svd_tol, cond_fp64, w, bt, st));
-    ISO_TRY(hipMemcpyAsync(rb, d.vbase, sizeof(int64_t) * (size_t) (n + 1), hipMemcpyDeviceToHost, st));
-    ISO_TRY(hipMemcpyAsync(rb + n + 1, d.qbase, sizeof(int64_t) * (size_t) (n + 1), hipMemcpyDeviceToHost, st));
-    ISO_TRY(hipMemcpyAsync(rb + 2 * n + 2, w.n_fp64, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+    // the totals, then the grids' first vertices and quads (adjacent)
+    ISO_TRY(hipMemcpyAsync(rb, w.tot, 5 * sizeof(int64_t), hipMemcpyDeviceToHost, st));
+    if (bt.vbase)
+        ISO_TRY(hipMemcpyAsync(rb + 5, d.vbase, sizeof(int64_t) * 2 * (size_t) (n + 1), hipMemcpyDeviceToHost, st));
     ISO_TRY(hipStreamSynchronize(st));
+    const int64_t *vb = rb + 5, *qb = vb + n + 1;
     for (int i = 0; i < n; ++i) {
-        nv[i] = rb[i + 1] - rb[i];
-        nq[i] = rb[n + 2 + i] - rb[n + 1 + i];
+        nv[i] = bt.vbase ? vb[i + 1] - vb[i] : rb[2];
+        nq[i] = bt.vbase ? qb[i + 1] - qb[i] : (tables ? rb[3] : rb[0]);
     }
-    w.nquads = rb[2 * n + 1];
-    n_fp64 = rb[2 * n + 2];
+    w.nquads = bt.vbase ? qb[n] : nq[0];
+    n_fp64 = rb[4];
     return hipSuccess;
 }
 
