@@ -206,6 +206,29 @@ int isoext_dc(const isoext_grid *g, const isoext_its *its, float reg, float svd_
               int64_t workspace_bytes, float *out_v, int64_t cap_v, int32_t *out_f, int64_t cap_f,
               float *dual_v, int32_t *out_vcell, int64_t counts[4], void *stream);
 
+/* isoext_its_count and isoext_its_emit of a dense grid without a gap on the
+ * device: begin launches the count and returns at once, finish (same thread,
+ * stream, grid, level and scratch) launches the rest into buffers of
+ * cap_cells (cell_offsets: cap_cells + 1) and cap_pts entries and waits for
+ * the counts only, {cells, points}.  On ISOEXT_E_CAPACITY they hold the need,
+ * and finish may be called again with more room. */
+int isoext_its_begin(const isoext_grid *g, float level, void *scratch, int64_t scratch_bytes, void *stream);
+int isoext_its_finish(const isoext_grid *g, float level, void *scratch, int64_t cap_cells, int64_t cap_pts,
+                      int64_t *cell_indices, int64_t *cell_dense, int64_t *cell_offsets, float *points,
+                      float *normals, uint8_t *edge_local, uint8_t *is_out, int32_t *entry_cell,
+                      uint64_t *amask_tab, int32_t *apre_tab, int64_t counts[2], void *stream);
+
+/* dual_contouring(grid, level) of a dense grid in one call with one
+ * synchronisation (no intersection set: trilinear normals).  Room for
+ * cap_cells active cells in the workspace, cap_v vertices and cap_f faces.
+ * counts = {vertices, faces, FP64 re-solves, active cells, intersections}; on
+ * ISOEXT_E_CAPACITY the active cells needed, and, where those fit, the
+ * vertices and faces. */
+int64_t isoext_dc_grid_workspace_bytes(const isoext_grid *g, int64_t cap_cells);
+int isoext_dc_grid(const isoext_grid *g, float level, float reg, float svd_tol, void *workspace,
+                   int64_t workspace_bytes, int64_t cap_cells, float *out_v, int64_t cap_v, int32_t *out_f,
+                   int64_t cap_f, int64_t counts[5], void *stream);
+
 /* Backward of dual contouring (no reference counterpart): accumulates
  * dL/dvalues += dL/dv * dv/dvalues through the regularised QEF solve of each
  * output vertex's cell and the edge interpolation of its intersection

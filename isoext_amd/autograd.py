@@ -101,10 +101,10 @@ class MarchingCubesFunction(torch.autograd.Function):
 class DualContouringFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, values, normals, grid, level, reg, svd_tol):
-        from .dc import compute_normals, dc_raw, get_intersection
+        from .dc import dc_raw, get_intersection
         vals = values.detach().contiguous()
         view = _View(grid, vals)
-        its = get_intersection(view, level, False)
+        its = get_intersection(view, level, normals is None)
         dev = vals.device
         if its.points.shape[0] == 0:
             ctx.empty = True
@@ -112,11 +112,12 @@ class DualContouringFunction(torch.autograd.Function):
             e = torch.empty((0, 3), dtype=torch.float32, device=dev)
             return e, torch.empty((0, 3), dtype=torch.int32, device=dev)
         ctx.empty = False
-        n = normals.detach().contiguous().float() if normals is not None else compute_normals(view, its)
+        n = normals.detach().contiguous().float() if normals is not None else its.normals
         v, f, info = dc_raw(view, its, n, reg, svd_tol, want_vcell=True)
         ctx.view, ctx.its, ctx.normals = view, its, n
         ctx.level, ctx.reg, ctx.svd_tol = float(level), float(reg), float(svd_tol)
         ctx.has_normals = normals is not None
+        ctx.set_materialize_grads(False)   # no gradient of the faces is made up
         ctx.save_for_backward(vals, info["vcell"])
         ctx.mark_non_differentiable(f)
         return v, f

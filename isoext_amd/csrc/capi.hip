@@ -351,6 +351,29 @@ DcLayout dc_layout(int64_t ncells, int64_t npts) {
     return L;
 }
 
+iso::DcScratch dc_scratch(char *ws, const DcLayout &L) {
+    iso::DcScratch w;
+    w.dual_v = (float *) (ws + L.o_dual);
+    w.cond = (float *) (ws + L.o_cond);
+    w.used = (uint8_t *) (ws + L.o_used);
+    w.bnd = (uint8_t *) (ws + L.o_bnd);
+    w.qn = (uint8_t *) (ws + L.o_qn);
+    w.qmask = (uint8_t *) (ws + L.o_qm);
+    w.bsum = (int64_t *) (ws + L.o_bsum);
+    w.part = (int64_t *) (ws + L.o_part);
+    w.tot = (int64_t *) (ws + L.o_tot);
+    w.n_fp64 = (unsigned long long *) (w.tot + 4);
+    w.tri_cells = (int32_t *) (ws + L.o_tri);
+    w.cap_tri = 6;
+    w.hslots = (uint32_t *) (ws + L.o_hs);
+    w.hmask = L.hslots - 1;
+    w.akey = (int64_t *) (ws + L.o_ak);
+    w.aval = (int32_t *) (ws + L.o_av);
+    w.amask = L.hslots - 1;
+    w.rep_slot = (int32_t *) (ws + L.o_rep);
+    w.final_id = (int32_t *) (ws + L.o_fin);
+    return w;
+}
 
 // ---- ragged batches of dense marching cubes --------------------------------------
 
@@ -703,6 +726,33 @@ DcBatchLayout dc_batch_layout(int n, const isoext_mc_item *items, int64_t C, int
 
 thread_local Pinned g_pinned_its;   // batched DC: intersection output descriptors
 
+// Counts of the calling thread's begun intersection set: they land in pinned
+// memory, the event says when.
+struct ItsPending {
+    hipEvent_t ev = nullptr;
+    int dev = -1;
+    int64_t *h = nullptr;
+    bool ready = false;
+    ~ItsPending() {
+        if (ev) (void) hipEventDestroy(ev);
+        if (h) (void) hipHostFree(h);
+    }
+    hipError_t prepare() {
+        int d = -1;
+        hipError_t e = hipGetDevice(&d);
+        if (e != hipSuccess) return e;
+        if (!h && (e = hipHostMalloc((void **) &h, 2 * sizeof(int64_t), 0)) != hipSuccess) return e;
+        if (ev && dev != d) {
+            (void) hipEventDestroy(ev);
+            ev = nullptr;
+        }
+        if (!ev && (e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) return e;
+        dev = d;
+        return hipSuccess;
+    }
+};
+thread_local ItsPending g_its_pending;
+
 }   // namespace
 
 extern "C" {
@@ -772,6 +822,125 @@ int isoext_its_emit(const isoext_grid *g, float level, const void *scratch, int6
     return ISOEXT_OK;
 }
 
+int isoext_its_begin(const isoext_grid *g, float level, void *scratch, int64_t scratch_bytes, void *stream) {
+    g_its_pending.ready = false;
+    AABB_CHECK(g->aabb_min, g->aabb_max);
+    if (g->sparse_cell_ids) return fail(ISOEXT_E_ARG, "isoext_its_begin takes dense grids");
+    if (!grid_has_cells(g)) return ISOEXT_OK;
+    if (scratch_bytes < isoext_its_scratch_bytes(g)) return fail(ISOEXT_E_WORKSPACE, "intersection scratch too small");
+    hipStream_t st = (hipStream_t) stream;
+    HIP_CHECK(g_its_pending.prepare(), "intersection count");
+    iso::McParams p = its_params(g, level, (char *) scratch, 0, 0);
+    HIP_CHECK(iso::its_dense_count_launch(p, st), "intersection count");
+    HIP_CHECK(hipMemcpyAsync(g_its_pending.h, p.totals, 2 * sizeof(int64_t), hipMemcpyDeviceToHost, st), "read counts");
+    HIP_CHECK(hipEventRecord(g_its_pending.ev, st), "intersection count");
+    g_its_pending.ready = true;
+    return ISOEXT_OK;
+}
+
+int isoext_its_finish(const isoext_grid *g, float level, void *scratch, int64_t cap_cells, int64_t cap_pts,
+                      int64_t *cell_indices, int64_t *cell_dense, int64_t *cell_offsets, float *points, float *normals,
+                      uint8_t *edge_local, uint8_t *is_out, int32_t *entry_cell, uint64_t *amask_tab,
+                      int32_t *apre_tab, int64_t counts[2], void *stream) {
+    counts[0] = counts[1] = 0;
+    hipStream_t st = (hipStream_t) stream;
+    if (!grid_has_cells(g)) {
+        HIP_CHECK(iso::fill_i64(cell_offsets, 1, 0, st), "write offsets");
+        return ISOEXT_OK;
+    }
+    if (!g_its_pending.ready) return fail(ISOEXT_E_ARG, "isoext_its_finish without isoext_its_begin");
+    iso::McParams p = its_params(g, level, (char *) scratch, cap_cells, cap_pts);
+    iso::ItsOut o{cell_indices, cell_dense, cell_offsets, points, normals, edge_local, is_out, entry_cell};
+    o.amask_tab = amask_tab;
+    o.apre_tab = apre_tab;
+    HIP_CHECK(iso::its_dense_emit_launch(iso::mc_auto_config(g->shape), p, o, st), "intersection emit");
+    HIP_CHECK(hipEventSynchronize(g_its_pending.ev), "intersection count");
+    counts[0] = g_its_pending.h[0];
+    counts[1] = g_its_pending.h[1];
+    if (counts[0] > 0x7fffffffll) return fail(ISOEXT_E_TOO_LARGE, "more than 2^31-1 active cells");
+    if (counts[0] > cap_cells || counts[1] > cap_pts)
+        return fail(ISOEXT_E_CAPACITY, "intersection buffers too small: need %lld cells, %lld points",
+                    (long long) counts[0], (long long) counts[1]);
+    return ISOEXT_OK;
+}
+
+// Scratch of isoext_dc_grid: the mask pipeline's, the active cells and their
+// lookup tables, the DC work arrays.
+struct DcGridLayout {
+    size_t o_its, o_cd, o_tm, o_tp, o_dc, total;
+    DcLayout dc;
+    DcGridLayout(const isoext_grid *g, int64_t cap_cells) {
+        size_t o = 0;
+        auto take = [&](size_t b) {
+            const size_t r = o;
+            o = align256(o + b);
+            return r;
+        };
+        const int64_t T = std::max<int64_t>(isoext_its_table_entries(g->shape), 1);
+        o_its = take((size_t) isoext_its_scratch_bytes(g));
+        o_cd = take(sizeof(int64_t) * (size_t) cap_cells);
+        o_tm = take(sizeof(uint64_t) * (size_t) T);
+        o_tp = take(sizeof(int32_t) * (size_t) T);
+        dc = dc_layout(cap_cells, 0);
+        o_dc = take(dc.total);
+        total = o;
+    }
+};
+
+int64_t isoext_dc_grid_workspace_bytes(const isoext_grid *g, int64_t cap_cells) {
+    if (!grid_has_cells(g) || g->sparse_cell_ids || cap_cells < 1) return 64;
+    return (int64_t) DcGridLayout(g, cap_cells).total;
+}
+
+int isoext_dc_grid(const isoext_grid *g, float level, float reg, float svd_tol, void *workspace,
+                   int64_t workspace_bytes, int64_t cap_cells, float *out_v, int64_t cap_v, int32_t *out_f,
+                   int64_t cap_f, int64_t counts[5], void *stream) {
+    for (int k = 0; k < 5; ++k) counts[k] = 0;
+    AABB_CHECK(g->aabb_min, g->aabb_max);
+    if (g->sparse_cell_ids) return fail(ISOEXT_E_ARG, "isoext_dc_grid takes dense grids");
+    for (int a = 0; a < 3; ++a)
+        if (g->shape[a] < 1) return fail(ISOEXT_E_ARG, "grid shape must be positive");
+    if (!grid_has_cells(g)) return ISOEXT_OK;
+    if (cap_cells < 1 || cap_cells > 0x3fffffffll) return fail(ISOEXT_E_ARG, "invalid cell capacity");
+    const DcGridLayout L(g, cap_cells);
+    if (workspace_bytes < (int64_t) L.total) return fail(ISOEXT_E_WORKSPACE, "dual contouring workspace too small");
+    hipStream_t st = (hipStream_t) stream;
+    int64_t *h = (int64_t *) g_pinned_its.get(8 * sizeof(int64_t));
+    if (!h) return fail(ISOEXT_E_DEVICE, "pinned staging allocation failed");
+    char *ws = (char *) workspace;
+    iso::McParams p = its_params(g, level, ws + L.o_its, cap_cells, INT64_MAX);
+    HIP_CHECK(iso::its_dense_count_launch(p, st), "intersection count");
+    iso::ItsOut o{};   // active cells and lookup tables only
+    o.cell_dense = (int64_t *) (ws + L.o_cd);
+    o.amask_tab = (uint64_t *) (ws + L.o_tm);
+    o.apre_tab = (int32_t *) (ws + L.o_tp);
+    HIP_CHECK(iso::its_dense_emit_launch(iso::mc_auto_config(g->shape), p, o, st), "active cells");
+    iso::DcScratch w = dc_scratch(ws + L.o_dc, L.dc);
+    w.out_v = out_v;
+    w.cap_v = cap_v;
+    w.out_f = out_f;
+    w.cap_q = cap_f / 2;
+    w.out_vcell = nullptr;
+    const float cond_fp64 = std::min(1e6f, 0.5f / std::max(svd_tol, 1e-30f));
+    HIP_CHECK(iso::dc_grid_launch(to_desc(g), level, o.cell_dense, cap_cells, p.totals, o.amask_tab, o.apre_tab, reg,
+                                  svd_tol, cond_fp64, w, st),
+              "dual contouring");
+    HIP_CHECK(hipMemcpyAsync(h, w.tot, 7 * sizeof(int64_t), hipMemcpyDeviceToHost, st), "read counts");
+    HIP_CHECK(hipStreamSynchronize(st), "dual contouring");
+    counts[0] = h[2];
+    counts[1] = 2 * h[3];
+    counts[2] = h[4];
+    counts[3] = h[5];
+    counts[4] = h[6];
+    if (h[5] > 0x3fffffffll || h[6] > 0x7fffffffll / 6)
+        return fail(ISOEXT_E_TOO_LARGE, "grid of %lld active cells / %lld intersections is too large", (long long) h[5],
+                    (long long) h[6]);
+    if (h[5] > cap_cells || h[2] > cap_v || h[3] > w.cap_q)
+        return fail(ISOEXT_E_CAPACITY, "buffers too small: %lld cells, %lld vertices, %lld faces", (long long) h[5],
+                    (long long) h[2], (long long) (2 * h[3]));
+    return ISOEXT_OK;
+}
+
 int isoext_dc_backward(const isoext_grid *g, const isoext_its *its, float reg, float svd_tol, float level,
                        int64_t nv, const int32_t *vcell, const float *grad_v, float *grad_values,
                        float *grad_normals, void *stream) {
@@ -803,26 +972,9 @@ int isoext_dc(const isoext_grid *g, const isoext_its *its, float reg, float svd_
     if (cap_v < its->ncells || cap_f < 2 * its->npts) return fail(ISOEXT_E_CAPACITY, "output capacity too small");
     hipStream_t st = (hipStream_t) stream;
     char *ws = (char *) workspace;
-    iso::DcScratch w;
-    w.dual_v = dual_v ? dual_v : (float *) (ws + L.o_dual);
-    w.cond = (float *) (ws + L.o_cond);
-    w.used = (uint8_t *) (ws + L.o_used);
-    w.bnd = (uint8_t *) (ws + L.o_bnd);
-    w.qn = (uint8_t *) (ws + L.o_qn);
-    w.qmask = (uint8_t *) (ws + L.o_qm);
-    w.bsum = (int64_t *) (ws + L.o_bsum);
-    w.part = (int64_t *) (ws + L.o_part);
-    w.tot = (int64_t *) (ws + L.o_tot);
-    w.n_fp64 = (unsigned long long *) (w.tot + 4);
-    w.tri_cells = (int32_t *) (ws + L.o_tri);
+    iso::DcScratch w = dc_scratch(ws, L);
+    if (dual_v) w.dual_v = dual_v;
     w.cap_tri = 6 * std::max<int64_t>(its->npts, 1);
-    w.hslots = (uint32_t *) (ws + L.o_hs);
-    w.hmask = L.hslots - 1;
-    w.akey = (int64_t *) (ws + L.o_ak);
-    w.aval = (int32_t *) (ws + L.o_av);
-    w.amask = L.hslots - 1;
-    w.rep_slot = (int32_t *) (ws + L.o_rep);
-    w.final_id = (int32_t *) (ws + L.o_fin);
     w.out_v = out_v;
     w.out_f = out_f;
     w.out_vcell = out_vcell;
@@ -1831,28 +1983,7 @@ int isoext_dc_batch_run(int n, const isoext_mc_item *items, const int64_t *count
     in.ncells = C;
     in.npts = P;
     in.cell_dense = (const int64_t *) (sc + L.o_cd);
-    char *dw = sc + L.o_dc;
-    const DcLayout &D = L.dc;
-    iso::DcScratch w;
-    w.dual_v = (float *) (dw + D.o_dual);
-    w.cond = (float *) (dw + D.o_cond);
-    w.used = (uint8_t *) (dw + D.o_used);
-    w.bnd = (uint8_t *) (dw + D.o_bnd);
-    w.qn = (uint8_t *) (dw + D.o_qn);
-    w.qmask = (uint8_t *) (dw + D.o_qm);
-    w.bsum = (int64_t *) (dw + D.o_bsum);
-    w.part = (int64_t *) (dw + D.o_part);
-    w.tot = (int64_t *) (dw + D.o_tot);
-    w.n_fp64 = (unsigned long long *) (w.tot + 4);
-    w.tri_cells = (int32_t *) (dw + D.o_tri);
-    w.cap_tri = 6;
-    w.hslots = (uint32_t *) (dw + D.o_hs);
-    w.hmask = D.hslots - 1;
-    w.akey = (int64_t *) (dw + D.o_ak);
-    w.aval = (int32_t *) (dw + D.o_av);
-    w.amask = D.hslots - 1;
-    w.rep_slot = (int32_t *) (dw + D.o_rep);
-    w.final_id = (int32_t *) (dw + D.o_fin);
+    iso::DcScratch w = dc_scratch(sc + L.o_dc, L.dc);
     w.out_v = out_v;
     w.out_f = out_f;
     w.out_vcell = nullptr;

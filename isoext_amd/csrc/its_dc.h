@@ -77,6 +77,7 @@ struct DcScratch {
     int32_t *aval;
     int64_t amask;
     float *out_v;
+    int64_t cap_v = INT64_MAX, cap_q = INT64_MAX;   // room for vertices and quads, where it may be short
     int32_t *out_f;
     int32_t *out_vcell;   // optional: active cell of each output vertex
     int64_t nquads;
@@ -92,6 +93,15 @@ hipError_t fill_i64(int64_t *p, int64_t n, int64_t v, hipStream_t st);
 // FP64 re-solves.
 hipError_t dc_run(const GridDesc &g, const ItsIn &in, float reg, float svd_tol, float cond_fp64, DcScratch &w,
                   int64_t &nv, int64_t &nf, int64_t &n_fp64, hipStream_t st);
+// Dual contouring of a dense grid without an intersection set, launched before
+// its active cells are counted on the host: count[0..1] on the device hold its
+// active cells and entries; at most `most` cells are worked on, more give
+// nothing.  Leaves w.tot[2] vertices, [3] quads, [4] FP64 re-solves, [5..6]
+// the counts; vertices past w.cap_v and quads past w.cap_q are not written.
+// No synchronisation.
+hipError_t dc_grid_launch(const GridDesc &g, float level, const int64_t *cell_dense, int64_t most,
+                          const int64_t *count, const uint64_t *amask, const int32_t *apre, float reg, float svd_tol,
+                          float cond_fp64, DcScratch &w, hipStream_t st);
 // Batched dual contouring of dense grids g[0, n) (n <= 256) whose
 // intersection sets are concatenated in `in` (grid i's active cells start at
 // cell0[i]; cell offsets and entry cells index the concatenated arrays).

@@ -288,6 +288,19 @@ struct DcBatch {
     int64_t *qbase;        // n + 1: first quad of each grid, total
 };
 
+// Active cells of a run: `most` given by the host, or, where it launches
+// before it knows (`count`), the device's count, 0 when that is above `most`
+// (the caller comes back with more room).
+struct CellCount {
+    int64_t most;
+    const int64_t *count;
+    __device__ __forceinline__ int64_t get() const {
+        if (!count) return most;
+        const int64_t n = *count;
+        return n <= most ? n : 0;
+    }
+};
+
 struct WeldClear {
     uint32_t *slots;
     int64_t hmask;
@@ -669,7 +682,7 @@ struct QefLdsEdges {
     }
 };
 
-__global__ void __launch_bounds__(64) k_dc_qef_grid(const int64_t *cell_dense, int64_t ncells, const CellSrc s1,
+__global__ void __launch_bounds__(64) k_dc_qef_grid(const int64_t *cell_dense, CellCount cells, const CellSrc s1,
                                                     float level, float reg, float svd_tol, float cond_fp64,
                                                     float *dual_v, uint8_t *used, uint8_t *bnd, uint8_t *qn,
                                                     uint8_t *qmask, DcBatch bt, WeldClear clr) {
@@ -678,6 +691,8 @@ __global__ void __launch_bounds__(64) k_dc_qef_grid(const int64_t *cell_dense, i
     const int c = threadIdx.x;
     const int64_t a = (int64_t) blockIdx.x * 64 + c;
     const CellSrc *sp = &s1;
+    const int64_t ncells = cells.get();
+    if ((int64_t) blockIdx.x * 64 >= ncells) return;
     bool mine = a < ncells;
     if (mine && bt.items) {
         // grids of one cell each are the rule in a wave: few steps, in the L2
@@ -1004,6 +1019,7 @@ struct WeldIds {
     const uint32_t *slots;
     const int32_t *final_id;
     int32_t *out_f;
+    int64_t cap_q;   // room for quads
 };
 __device__ __forceinline__ int32_t welded_id(const WeldIds &wd, int32_t a) {
     return wd.final_id[(wd.bnd[a] & kOnBox) ? (int32_t) wd.slots[wd.rep_slot[a]] : a];
@@ -1061,10 +1077,10 @@ __global__ void k_quad_emit(ItsIn in, CellSrc s1, ActHash ah, const int64_t *bsu
 
 // A slot holds the lowest cell at its position (all ones: empty): whichever
 // cell of a position arrives first claims the slot, the others lower it.
-__global__ void k_pos_insert(const float *dv, const uint8_t *used, const uint8_t *bnd, int64_t n, uint32_t *slots,
-                             int64_t mask, int32_t *rep, const int32_t *cell_item) {
+__global__ void k_pos_insert(const float *dv, const uint8_t *used, const uint8_t *bnd, CellCount cells,
+                             uint32_t *slots, int64_t mask, int32_t *rep, const int32_t *cell_item) {
     int64_t a = (int64_t) blockIdx.x * kBlock + threadIdx.x;
-    if (a >= n || !used[a] || !(bnd[a] & kOnBox)) return;
+    if (a >= cells.get() || !used[a] || !(bnd[a] & kOnBox)) return;
     float x = dv[3 * a], y = dv[3 * a + 1], z = dv[3 * a + 2];
     // batches: vertices of different grids never weld (the grid joins the hash and the test)
     const int32_t item = cell_item ? cell_item[a] : 0;
@@ -1124,9 +1140,13 @@ __device__ __forceinline__ void block_base(const int64_t *bsum, bool scanned, in
 }
 
 // Block sums of (kept vertices, quads per cell from qn, or 0 without it).
-// The FP64 re-solves are counted on the way.
-__global__ void k_keep_flags(const uint8_t *used, const uint8_t *bnd, int64_t n, const int32_t *rep_slot,
-                             const uint32_t *slots, const uint8_t *qn, int64_t *bsum, unsigned long long *n_fp64) {
+// The FP64 re-solves are counted on the way; a device-side count's cells and
+// entries go to its[0..1], for one read-back at the end.
+__global__ void k_keep_flags(const uint8_t *used, const uint8_t *bnd, CellCount cells, const int32_t *rep_slot,
+                             const uint32_t *slots, const uint8_t *qn, int64_t *bsum, unsigned long long *n_fp64,
+                             int64_t *its) {
+    const int64_t n = cells.get();
+    if (cells.count && blockIdx.x == 0 && threadIdx.x < 2) its[threadIdx.x] = cells.count[threadIdx.x];
     int64_t a = (int64_t) blockIdx.x * kBlock + threadIdx.x;
     int64_t k = (a < n && kept_vertex(used, bnd, rep_slot, slots, a)) ? 1 : 0;
     int64_t q = (qn && a < n) ? qn[a] : 0;
@@ -1142,9 +1162,11 @@ __global__ void k_keep_flags(const uint8_t *used, const uint8_t *bnd, int64_t n,
 
 // tot (optional): the totals, left by the last block where the sums are not
 // scanned.
-__global__ void k_keep_emit(const float *dv, const uint8_t *used, const uint8_t *bnd, int64_t n,
+__global__ void k_keep_emit(const float *dv, const uint8_t *used, const uint8_t *bnd, CellCount cells,
                             const int32_t *rep_slot, const uint32_t *slots, const int64_t *bsum, bool scanned,
-                            int64_t *tot, int32_t *final_id, float *out_v, int32_t *out_vcell, DcBatch bt) {
+                            int64_t *tot, int32_t *final_id, float *out_v, int64_t cap_v, int32_t *out_vcell,
+                            DcBatch bt) {
+    const int64_t n = cells.get();
     int64_t a = (int64_t) blockIdx.x * kBlock + threadIdx.x;
     int64_t k = (a < n && kept_vertex(used, bnd, rep_slot, slots, a)) ? 1 : 0;
     int64_t ek, d, tk, td, bv, bq;
@@ -1154,6 +1176,7 @@ __global__ void k_keep_emit(const float *dv, const uint8_t *used, const uint8_t 
     const int64_t id = bv + ek;
     // batch: face corners use grid-local vertex ids
     final_id[a] = (int32_t) (bt.vbase ? id - bt.vbase[bt.cell_item[a]] : id);
+    if (id >= cap_v) return;
     out_v[3 * id + 0] = dv[3 * a + 0];
     out_v[3 * id + 1] = dv[3 * a + 1];
     out_v[3 * id + 2] = dv[3 * a + 2];
@@ -1252,16 +1275,17 @@ __device__ __forceinline__ void grid_quad(const CellSrc &s, const uint64_t *amas
     for (int k = 0; k < 6; ++k) wd.out_f[6 * slot + k] = t[k];
 }
 
-__global__ void k_quad_emit_grid(const int64_t *cell_dense, int64_t ncells, CellSrc s1, const uint64_t *amask_tab,
+__global__ void k_quad_emit_grid(const int64_t *cell_dense, CellCount cells, CellSrc s1, const uint64_t *amask_tab,
                                  const int32_t *apre_tab, const uint8_t *qn, const uint8_t *qmask,
                                  const int64_t *bsum, bool scanned, const float *dual_v, WeldIds wd, DcBatch bt) {
     const int64_t a = (int64_t) blockIdx.x * kBlock + threadIdx.x;
-    const int64_t nq = a < ncells ? qn[a] : 0;
+    const int64_t nq = a < cells.get() ? qn[a] : 0;
     int64_t ed, eq, td, tq, bv, bq;
     block_base(bsum, scanned, nullptr, bv, bq);
     block_scan2(0, nq, ed, eq, td, tq);
     if (!nq) return;
     int64_t slot = bq + eq;
+    if (slot + nq > wd.cap_q) return;
     const DcItem *it = bt.items ? &bt.items[bt.cell_item[a]] : nullptr;
     const CellSrc &s = it ? it->s : s1;
     const uint64_t *am = it ? it->amask : amask_tab;
@@ -1575,25 +1599,25 @@ static void scan_pairs(int64_t *bsum, int64_t nb, int64_t *tot, int64_t *part, h
 
 // Weld, vertex and quad offsets, vertices, faces.  Leaves the totals in
 // w.tot[2] (vertices) and, with tables (dense grids), w.tot[3] (quads).
-static void weld_and_emit(const CellSrc &s, const ItsIn &in, const uint64_t *amask, const int32_t *apre, bool tables,
-                          DcScratch &w, const DcBatch &bt, hipStream_t st) {
+static void weld_and_emit(const CellSrc &s, const ItsIn &in, const CellCount &cells, const uint64_t *amask,
+                          const int32_t *apre, bool tables, DcScratch &w, const DcBatch &bt, hipStream_t st) {
     const unsigned nbv = nblocks(in.ncells);
-    const WeldIds wd{w.bnd, w.rep_slot, w.hslots, w.final_id, w.out_f};
+    const WeldIds wd{w.bnd, w.rep_slot, w.hslots, w.final_id, w.out_f, w.cap_q};
     const uint8_t *qn = tables ? w.qn : nullptr;
-    hipLaunchKernelGGL(k_pos_insert, dim3(nbv), dim3(kBlock), 0, st, w.dual_v, w.used, w.bnd, in.ncells, w.hslots,
+    hipLaunchKernelGGL(k_pos_insert, dim3(nbv), dim3(kBlock), 0, st, w.dual_v, w.used, w.bnd, cells, w.hslots,
                        w.hmask, w.rep_slot, (const int32_t *) bt.cell_item);
-    hipLaunchKernelGGL(k_keep_flags, dim3(nbv), dim3(kBlock), 0, st, w.used, w.bnd, in.ncells, w.rep_slot, w.hslots,
-                       qn, w.bsum, w.n_fp64);
+    hipLaunchKernelGGL(k_keep_flags, dim3(nbv), dim3(kBlock), 0, st, w.used, w.bnd, cells, w.rep_slot, w.hslots, qn,
+                       w.bsum, w.n_fp64, w.tot + 5);
     // several grids need the offsets of their first cells: scanned apart
     const bool scanned = bt.vbase || nbv > kDirectBlocks;
     if (scanned) scan_pairs(w.bsum, (int64_t) nbv, w.tot + 2, w.part, st);
     if (bt.vbase)
         hipLaunchKernelGGL(k_item_vbase, dim3(bt.n), dim3(kBlock), 0, st, bt, w.used, w.bnd, w.rep_slot, w.hslots, qn,
                            w.bsum, in.ncells, (const int64_t *) w.tot);
-    hipLaunchKernelGGL(k_keep_emit, dim3(nbv), dim3(kBlock), 0, st, w.dual_v, w.used, w.bnd, in.ncells, w.rep_slot,
-                       w.hslots, (const int64_t *) w.bsum, scanned, w.tot + 2, w.final_id, w.out_v, w.out_vcell, bt);
+    hipLaunchKernelGGL(k_keep_emit, dim3(nbv), dim3(kBlock), 0, st, w.dual_v, w.used, w.bnd, cells, w.rep_slot,
+                       w.hslots, (const int64_t *) w.bsum, scanned, w.tot + 2, w.final_id, w.out_v, w.cap_v, w.out_vcell, bt);
     if (tables)
-        hipLaunchKernelGGL(k_quad_emit_grid, dim3(nbv), dim3(kBlock), 0, st, in.cell_dense, in.ncells, s, amask, apre,
+        hipLaunchKernelGGL(k_quad_emit_grid, dim3(nbv), dim3(kBlock), 0, st, in.cell_dense, cells, s, amask, apre,
                            (const uint8_t *) w.qn, (const uint8_t *) w.qmask, (const int64_t *) w.bsum, scanned,
                            w.dual_v, wd, bt);
     else
@@ -1625,21 +1649,22 @@ static hipError_t dc_launch(const CellSrc &s, const ItsIn &in, float reg, float 
                            w.used, bt);
         if (bt.items) hipLaunchKernelGGL(k_item_qbase, dim3(1), dim3(64), 0, st, bt, in.ncells, (const int64_t *) w.tot);
     }
-    weld_and_emit(s, in, in.amask_tab, in.apre_tab, tables, w, bt, st);
+    weld_and_emit(s, in, CellCount{in.ncells, nullptr}, in.amask_tab, in.apre_tab, tables, w, bt, st);
     return hipGetLastError();
 }
 
 // Dense grids without an intersection set (active cells and lookup tables
 // only): QEF from the corner values, weld, one scan for vertex and quad
 // offsets, quads per cell.
-static hipError_t dc_launch_grid(const CellSrc &s, const int64_t *cell_dense, int64_t ncells, const uint64_t *amask,
-                                 const int32_t *apre, float level, float reg, float svd_tol, float cond_fp64,
+static hipError_t dc_launch_grid(const CellSrc &s, const int64_t *cell_dense, const CellCount &cells,
+                                 const uint64_t *amask, const int32_t *apre, float level, float reg, float svd_tol, float cond_fp64,
                                  DcScratch &w, const DcBatch &bt, hipStream_t st, bool has_grid = true,
                                  bool has_prog = false) {
+    const int64_t ncells = cells.most;
     const unsigned nbv = nblocks(ncells);
     const WeldClear clr{w.hslots, w.hmask, w.n_fp64};
     if (has_grid)
-        hipLaunchKernelGGL(k_dc_qef_grid, dim3((unsigned) ((ncells + 63) / 64)), dim3(64), 0, st, cell_dense, ncells, s, level, reg,
+        hipLaunchKernelGGL(k_dc_qef_grid, dim3((unsigned) ((ncells + 63) / 64)), dim3(64), 0, st, cell_dense, cells, s, level, reg,
                            svd_tol, cond_fp64, w.dual_v, w.used, w.bnd, w.qn, w.qmask, bt, clr);
     if (has_prog)
         hipLaunchKernelGGL(k_dc_qef_prog, dim3(nbv), dim3(kBlock), 0, st, cell_dense, ncells, s, level, reg,
@@ -1647,7 +1672,7 @@ static hipError_t dc_launch_grid(const CellSrc &s, const int64_t *cell_dense, in
     ItsIn in{};
     in.ncells = ncells;
     in.cell_dense = cell_dense;
-    weld_and_emit(s, in, amask, apre, true, w, bt, st);
+    weld_and_emit(s, in, cells, amask, apre, true, w, bt, st);
     return hipGetLastError();
 }
 
@@ -1675,6 +1700,13 @@ hipError_t dc_run(const GridDesc &g, const ItsIn &in, float reg, float svd_tol, 
     nf = 2 * nq;
     n_fp64 = pt.p[4];
     return hipSuccess;
+}
+
+hipError_t dc_grid_launch(const GridDesc &g, float level, const int64_t *cell_dense, int64_t most,
+                          const int64_t *count, const uint64_t *amask, const int32_t *apre, float reg, float svd_tol,
+                          float cond_fp64, DcScratch &w, hipStream_t st) {
+    return dc_launch_grid(make_src(g), cell_dense, CellCount{most, count}, amask, apre, level, reg, svd_tol, cond_fp64, w,
+                          DcBatch{}, st);
 }
 
 size_t dc_batch_item_bytes() { return sizeof(DcItem); }
@@ -1728,8 +1760,8 @@ hipError_t dc_run_batch(int n, const GridDesc *g, const int64_t *cell0, const ui
     // one grid starts at vertex 0 and quad 0
     const DcBatch bt{(const DcItem *) d.items, n, tables, d.cell_item, n > 1 ? d.vbase : nullptr, d.qbase};
     if (levels)
-        ISO_TRY(dc_launch_grid(hi[0].s, in.cell_dense, in.ncells, nullptr, nullptr, 0.0f, reg, svd_tol, cond_fp64, w,
-                               bt, st, has_grid, has_prog));
+        ISO_TRY(dc_launch_grid(hi[0].s, in.cell_dense, CellCount{in.ncells, nullptr}, nullptr, nullptr, 0.0f, reg, svd_tol,
+                               cond_fp64, w, bt, st, has_grid, has_prog));
     else
         ISO_TRY(dc_launch(hi[0].s, in, reg, svd_tol, cond_fp64, w, bt, st));
     // the totals, then the grids' first vertices and quads (adjacent)

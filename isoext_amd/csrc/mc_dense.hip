@@ -2193,6 +2193,9 @@ __device__ __forceinline__ void its_tile(const McParams &p, const ItsOut &o, int
 
 template <int TX, int TY, int NZC, int NT>
 __global__ void __launch_bounds__(NT) k_its_tiles(McParams p, ItsOut o) {
+    // the offset past the last cell, where there is room for all of them
+    if (o.cell_offsets && blockIdx.x == 0 && threadIdx.x == 0 && p.totals[0] <= p.cap_v)
+        o.cell_offsets[p.totals[0]] = p.totals[1];
     const int64_t tile = emit_block_tile(p);
     if (tile >= 0) its_tile<TX, TY, NZC, NT>(p, o, tile);
 }

@@ -22,6 +22,7 @@ Differences on purpose:
 from __future__ import annotations
 
 import ctypes
+import threading
 
 import torch
 
@@ -49,6 +50,11 @@ _lib.declare("isoext_its_count", ctypes.c_int, [P(IsoGrid), f32, vp, i64, i64 * 
 _lib.declare("isoext_its_table_entries", i64, [i64 * 3])
 _lib.declare("isoext_its_emit", ctypes.c_int, [P(IsoGrid), f32, vp, i64, i64, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp,
                                                vp])
+_lib.declare("isoext_its_begin", ctypes.c_int, [P(IsoGrid), f32, vp, i64, vp])
+_lib.declare("isoext_its_finish", ctypes.c_int, [P(IsoGrid), f32, vp, i64, i64, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp,
+                                                 i64 * 2, vp])
+_lib.declare("isoext_dc_grid_workspace_bytes", i64, [P(IsoGrid), i64])
+_lib.declare("isoext_dc_grid", ctypes.c_int, [P(IsoGrid), f32, f32, f32, vp, i64, i64, vp, i64, vp, i64, i64 * 5, vp])
 _lib.declare("isoext_its_normals", ctypes.c_int, [P(IsoGrid), P(IsoIts), vp, vp])
 _lib.declare("isoext_dc_workspace_bytes", i64, [i64, i64])
 _lib.declare("isoext_dc", ctypes.c_int, [P(IsoGrid), P(IsoIts), f32, f32, vp, i64, vp, i64, vp, i64, vp, vp,
@@ -150,37 +156,87 @@ def get_intersection(grid, level: float = 0.0, compute_normals: bool = False) ->
     dev = _device(grid)
     L = _lib.lib()
     g = grid_struct(grid)
-    nbytes = L.isoext_its_scratch_bytes(ctypes.byref(g))
+    nbytes = L.isoext_its_scratch_bytes(ctypes.byref(g)) if g.values else 64
     scratch = workspace.get("its", nbytes, dev)
     counts = (ctypes.c_int64 * 2)()
+    tables = None
     with torch.cuda.device(dev):
         stream = _lib.stream_ptr(dev)
-        _lib.check(L.isoext_its_count(ctypes.byref(g), float(level), scratch.data_ptr(), scratch.numel(), counts,
-                                      stream), "get_intersection")
-        nc, npt = int(counts[0]), int(counts[1])
-        i64t = dict(dtype=torch.int64, device=dev)
-        cell_indices = torch.empty(nc, **i64t)
-        cell_dense = torch.empty(nc, **i64t)
-        cell_offsets = torch.empty(nc + 1, **i64t)
-        points = torch.empty((npt, 3), dtype=torch.float32, device=dev)
-        normals = torch.empty((npt, 3), dtype=torch.float32, device=dev) if compute_normals else None
-        edge_local = torch.empty(npt, dtype=torch.uint8, device=dev)
-        is_out = torch.empty(npt, dtype=torch.uint8, device=dev)
-        entry_cell = torch.empty(npt, dtype=torch.int32, device=dev)
-        tables = None
-        if not g.sparse_cell_ids and nc > 0:
-            nt = int(L.isoext_its_table_entries(g.shape))
+        if getattr(grid, "cell_ids", None) is None:
+            # dense: the buffers, sized by the last set of this shape, are made while the count runs, and only the
+            # counts are waited for
+            _lib.check(L.isoext_its_begin(ctypes.byref(g), float(level), scratch.data_ptr(), scratch.numel(), stream),
+                       "get_intersection")
+            shape = tuple(g.shape)
+            nt = max(int(L.isoext_its_table_entries(g.shape)), 1)
             tables = (torch.empty(nt, dtype=torch.int64, device=dev), torch.empty(nt, dtype=torch.int32, device=dev))
-        _lib.check(L.isoext_its_emit(ctypes.byref(g), float(level), scratch.data_ptr(), nc, npt,
-                                     cell_indices.data_ptr(), cell_dense.data_ptr(), cell_offsets.data_ptr(),
-                                     points.data_ptr() if npt else None,
-                                     normals.data_ptr() if (normals is not None and npt) else None,
-                                     edge_local.data_ptr() if npt else None, is_out.data_ptr() if npt else None,
-                                     entry_cell.data_ptr() if npt else None,
-                                     tables[0].data_ptr() if tables else None,
-                                     tables[1].data_ptr() if tables else None, stream), "get_intersection")
+            nc, npt = _its_caps(shape)
+            for _ in range(2):
+                b = _its_buffers(nc, npt, compute_normals, dev)
+                rc = L.isoext_its_finish(ctypes.byref(g), float(level), scratch.data_ptr(), nc, npt,
+                                         *(t.data_ptr() if t is not None else None for t in b), tables[0].data_ptr(),
+                                         tables[1].data_ptr(), counts, stream)
+                if rc != _lib.E_CAPACITY:
+                    break
+                nc, npt = int(counts[0]), int(counts[1])
+            _lib.check(rc, "get_intersection")
+            cap, nc, npt = npt, int(counts[0]), int(counts[1])
+            with _hint_lock:
+                if len(_its_hint) > 4096:
+                    _its_hint.clear()
+                _its_hint[shape] = (nc, npt)
+            ends = (nc, nc, nc + 1, npt, npt, npt, npt, npt)
+            b = [t[:n] if t is not None else None for t, n in zip(b, ends)]
+            if cap > 2 * npt + 65536:   # do not pin much larger buffers behind a small set
+                b = [t.clone() if t is not None else None for t in b]
+            tables = tables if nc else None
+        elif g.n_sparse == 0:
+            b = _its_buffers(0, 0, compute_normals, dev)
+            b[2].zero_()
+        else:
+            _lib.check(L.isoext_its_count(ctypes.byref(g), float(level), scratch.data_ptr(), scratch.numel(), counts,
+                                          stream), "get_intersection")
+            nc, npt = int(counts[0]), int(counts[1])
+            b = _its_buffers(nc, npt, compute_normals, dev)
+            p = [t.data_ptr() if t is not None and (npt or k < 3) else None for k, t in enumerate(b)]
+            _lib.check(L.isoext_its_emit(ctypes.byref(g), float(level), scratch.data_ptr(), nc, npt, *p, None, None,
+                                         stream), "get_intersection")
+    cell_indices, cell_dense, cell_offsets, points, normals, edge_local, is_out, entry_cell = b
     return Intersection(grid, level, cell_indices, cell_dense, cell_offsets, points, normals, edge_local, is_out,
                         entry_cell, tables)
+
+
+# cells and points of the last intersection set of a dense shape, and cells and
+# faces of its last dual mesh (sizing hints)
+_its_hint: dict = {}
+_dc_hint: dict = {}
+_hint_lock = threading.Lock()
+
+
+def _its_caps(shape):
+    hint = _its_hint.get(shape)   # a single dict read needs no lock
+    if hint is None:
+        # surface-like: a few times the largest cross-section
+        X, Y, Z = shape
+        cells = min(max(1 << 15, 2 * max(X * Y, Y * Z, X * Z)), 0x3fffffff)
+        return cells, 4 * cells
+    return hint[0] + hint[0] // 8 + 1024, hint[1] + hint[1] // 8 + 4096
+
+
+def _dc_caps(shape):
+    hint = _dc_hint.get(shape)
+    if hint is None:
+        nc = _its_caps(shape)[0]
+        return nc, nc, 2 * nc
+    return tuple(min(n + n // 8 + 1024, m) for n, m in zip(hint, (0x3fffffff, 1 << 31, 1 << 32)))
+
+
+def _its_buffers(nc, npt, normals, dev):
+    """Cell indices, dense ids, offsets, points, normals, local edges, orientations, entry cells."""
+    i64t, f32t, u8t = (dict(dtype=t, device=dev) for t in (torch.int64, torch.float32, torch.uint8))
+    return [torch.empty(nc, **i64t), torch.empty(nc, **i64t), torch.empty(nc + 1, **i64t),
+            torch.empty((npt, 3), **f32t), torch.empty((npt, 3), **f32t) if normals else None, torch.empty(npt, **u8t),
+            torch.empty(npt, **u8t), torch.empty(npt, dtype=torch.int32, device=dev)]
 
 
 def compute_normals(grid, its: Intersection) -> torch.Tensor:
@@ -247,9 +303,7 @@ def dual_contouring(grid, level: float = 0.0, intersection: Intersection | None 
     """
     from .grid import UniformGrid
     if intersection is None and isinstance(grid, UniformGrid):
-        from .batch import GridJob, dc_batch
-        job = GridJob(grid.values, float(level), 0, tuple(grid.aabb_min), tuple(grid.aabb_max))
-        return dc_batch([job], reg=reg, svd_tol=svd_tol, ws_kind="dc_grid")[0]
+        return _dc_grid(grid, level, reg, svd_tol)
     its = intersection if intersection is not None else get_intersection(grid, level, True)
     if its.points.shape[0] == 0:
         return None, None
@@ -257,4 +311,45 @@ def dual_contouring(grid, level: float = 0.0, intersection: Intersection | None 
     v, f, _ = dc_raw(grid, its, normals.contiguous(), reg, svd_tol)
     if f.shape[0] == 0:
         return None, None
+    return v, f
+
+
+def _dc_grid(grid, level: float, reg: float, svd_tol: float):
+    """dual_contouring of a dense grid without an intersection set, into
+    buffers sized by the last mesh of this shape (one synchronisation)."""
+    check_cuda_f32(grid.values, 3, name="values")
+    dev = _device(grid)
+    L = _lib.lib()
+    g = grid_struct(grid)
+    shape = tuple(g.shape)
+    nc, cap_v, cap_f = _dc_caps(shape)
+    counts = (ctypes.c_int64 * 5)()
+    with torch.cuda.device(dev):
+        stream = _lib.stream_ptr(dev)
+        for _ in range(3):
+            ws = workspace.get("dc_grid", L.isoext_dc_grid_workspace_bytes(ctypes.byref(g), nc), dev, stream)
+            out_v = torch.empty((cap_v, 3), dtype=torch.float32, device=dev)
+            out_f = torch.empty((cap_f, 3), dtype=torch.int32, device=dev)
+            rc = L.isoext_dc_grid(ctypes.byref(g), float(level), float(reg), float(svd_tol), ws.data_ptr(), ws.numel(),
+                                  nc, out_v.data_ptr(), cap_v, out_f.data_ptr(), cap_f, counts, stream)
+            if rc != _lib.E_CAPACITY:
+                break
+            if counts[3] > nc:   # cells did not fit: a vertex each at most, and a quad per canonical edge, about as many
+                nc = int(counts[3])
+                cap_v, cap_f = nc, max(cap_f, 2 * nc)
+            else:
+                cap_v, cap_f = max(cap_v, int(counts[0])), max(cap_f, int(counts[1]))
+    _lib.check(rc, "dual_contouring")
+    nv, nf = int(counts[0]), int(counts[1])
+    with _hint_lock:
+        if len(_dc_hint) > 4096:
+            _dc_hint.clear()
+        _dc_hint[shape] = (int(counts[3]), nv, nf)
+    if nf == 0:
+        return None, None
+    v, f = out_v[:nv], out_f[:nf]
+    if cap_v > 2 * nv + 65536:   # do not pin a much larger allocation behind a small mesh
+        v = v.clone()
+    if cap_f > 2 * nf + 65536:
+        f = f.clone()
     return v, f
