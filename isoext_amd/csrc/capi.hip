@@ -85,7 +85,7 @@ struct McLayout {
 };
 
 constexpr size_t kHeader = 4096;   // err, totals, SpecialLists
-constexpr size_t kOffErr = 8, kOffTotals = 16, kOffSp = 64;
+constexpr size_t kOffErr = 8, kOffTotals = 16, kOffAny = 32, kOffSp = 64;
 
 size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
@@ -1296,6 +1296,18 @@ static int mc_dense_impl(const float *values, const int64_t shape[3], const floa
         p.csg = csg;
         p.csg_list = iso::csg_list_fits(p.X, p.Y, p.W, p.S) ? 1 : 0;
     }
+    // a plain call's last kernel writes what the host reads back; a captured
+    // plan, the allocation-free call and the read-once pipeline copy the header
+    const bool direct = !na && !plan && !L.stream;
+    iso::McHostResult *hres = nullptr;
+    if (!L.stream) p.sp_any = (int *) (ws + kOffAny);
+    if (direct) {
+        hres = (iso::McHostResult *) g_pinned_rb.get(sizeof(iso::McHostResult));
+        if (!hres) return fail(ISOEXT_E_DEVICE, "pinned read-back allocation failed");
+        hres->sp = sp_host;
+        hres->sp.dup = p.dslots ? 0 : -1;
+        p.host = hres;
+    }
     hipEvent_t *ev = (g_timing && !na && !plan) ? timing_events() : nullptr;
     if (g_timing && !na && !plan && !ev) return fail(ISOEXT_E_DEVICE, "timing events unavailable");
     if (plan && L.stream) return fail(ISOEXT_E_ARG, "plans take the four-stage tile configurations, not %d", cfg);
@@ -1353,14 +1365,20 @@ static int mc_dense_impl(const float *values, const int64_t shape[3], const floa
     static_assert(kOffTotals == kOffErr + 8 && kOffSp >= kOffErr + (int) sizeof(Header), "header layout");
     const size_t rb_bytes = kOffSp - kOffErr + sizeof(iso::SpecialLists);
     alignas(64) char rb_stack[kOffSp + sizeof(iso::SpecialLists)];
-    char *rb = na ? rb_stack : (char *) g_pinned_rb.get(rb_bytes);
-    if (!rb) return fail(ISOEXT_E_DEVICE, "pinned read-back allocation failed");
-    HIP_CHECK(hipMemcpyAsync(rb, ws + kOffErr, rb_bytes, hipMemcpyDeviceToHost, st), "read counts");
-    HIP_CHECK(hipStreamSynchronize(st), "marching cubes");
     Header hdr;
     iso::SpecialLists sp_dev;
-    std::memcpy(&hdr, rb, sizeof(hdr));
-    std::memcpy(&sp_dev, rb + (kOffSp - kOffErr), sizeof(sp_dev));
+    if (direct) {
+        HIP_CHECK(hipStreamSynchronize(st), "marching cubes");
+        hdr = Header{hres->err, 0, {hres->totals[0], hres->totals[1]}};
+        sp_dev = hres->sp;
+    } else {
+        char *rb = na ? rb_stack : (char *) g_pinned_rb.get(rb_bytes);
+        if (!rb) return fail(ISOEXT_E_DEVICE, "pinned read-back allocation failed");
+        HIP_CHECK(hipMemcpyAsync(rb, ws + kOffErr, rb_bytes, hipMemcpyDeviceToHost, st), "read counts");
+        HIP_CHECK(hipStreamSynchronize(st), "marching cubes");
+        std::memcpy(&hdr, rb, sizeof(hdr));
+        std::memcpy(&sp_dev, rb + (kOffSp - kOffErr), sizeof(sp_dev));
+    }
     if (ev) {
         float ms[5] = {-1.0f, -1.0f, -1.0f, -1.0f, -1.0f};
         for (int i = 0; i < 4; ++i) (void) hipEventElapsedTime(&ms[i], ev[i], ev[i + 1]);

@@ -71,6 +71,14 @@ constexpr int kMcScanBlock = 1024;
 constexpr int kFlatChunks = 32;
 constexpr int64_t kFlatPts = 64 * kFlatChunks;
 
+// What a single-grid call reads back, in pinned host memory that the last
+// kernel writes: no copy launch.
+struct McHostResult {
+    int err, pad;
+    int64_t totals[2];
+    SpecialLists sp;   // capacities and pointers by the host, counts, need and dup by the device
+};
+
 struct McParams {
     const float *values;
     int64_t X, Y, Z;   // points per axis
@@ -101,6 +109,8 @@ struct McParams {
     int64_t *totals;    // [0] vertices, [1] faces (provisional)
     SpecialLists *sp;   // contiguous lists (written by the gather pass)
     SpecialSegs seg;    // segmented lists (written by emit)
+    int *sp_any;        // optional: set when emit appends a special entry (cleared by the reset)
+    McHostResult *host;   // optional: read-back written by the gather
     // fused field (values unused when nsph > 0): v(p) = min_k |p - c_k| - r_k
     // over nsph <= kMaxFusedSpheres spheres (cx, cy, cz, r), evaluated where
     // needed with the sphere-union generator's formula

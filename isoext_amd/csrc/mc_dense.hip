@@ -56,6 +56,7 @@ static __constant__ uint8_t cNtri[2][256];   // triangles per case (the low 4 bi
 // Returns the entry index, or -1 when the segment is full (the counter
 // still counts so the host can size a retry).
 __device__ __forceinline__ int64_t seg_push(const McParams &p, int k, int seg) {
+    if (p.sp_any) *p.sp_any = 1;   // any lane, the same value
     seg = (seg + (int) threadIdx.x) & (p.seg.nseg - 1);   // nseg: a power of two
     const unsigned long long i = atomicAdd(&p.seg.ctr[(k * p.seg.nseg + seg) * kSpStride], 1ull);
     return (int64_t) i < p.seg.cap[k] ? (int64_t) seg * p.seg.cap[k] + (int64_t) i : -1;
@@ -76,6 +77,7 @@ __device__ __forceinline__ void reset_state(const McParams &p, SpecialLists init
         for (int64_t i = t; i <= p.dmask; i += stride) p.dslots[i] = -1;
     if (t == 0) {
         if (p.tile_count) *p.tile_count = 0;
+        if (p.sp_any) *p.sp_any = 0;
         if (p.csg) p.cnt_f[0] = 0;   // the program classify's block list count
         *p.err = 0;
         p.totals[0] = p.totals[1] = 0;
@@ -1135,33 +1137,25 @@ __device__ __forceinline__ bool edge_maybe_candidate(const CellCtx &cc, float ep
 }
 
 template <int TX, int TY, int NZC, int NT, int SRC = kSrcGrid>
-__device__ __forceinline__ void emit_tile(const McParams &p, int64_t tile, int spseg) {
+__device__ __forceinline__ void emit_tile(const McParams &p, int64_t tile, int spseg, int sum_v = 0, int sum_f = 0) {
     using L = EmitLds<TX, TY, NZC, NT>;
     __shared__ L s;
     __shared__ FusedLds<SRC, NZC> fl;
     __shared__ CsgTileCache<TX, TY, NZC, SRC == kSrcProgram> cache;
     const int tid = threadIdx.x;
-    if (*(volatile int *) p.err & ISO_ERR_TOO_LARGE) return;
-
-    // small grids (nblk <= NT): the block totals are scanned here, into the
-    // LDS of the id table (used only by the batches below, after the bases
-    // are read); workgroup 0 also publishes the bases and the mesh size
+    // small grids (nblk <= NT): the block totals (sum_v, sum_f: this lane's
+    // block, loaded with the tile's number) are scanned here, into the LDS of
+    // the id table (used only by the batches below, after the bases are read);
+    // workgroup 0 also publishes the bases and the mesh size.  256 blocks of
+    // 1024 entries of at most 512 cells and 5 faces each: below 2^31.
     const int64_t *bv_tab = p.blk_v, *bf_tab = p.blk_f;
     if (p.scan_in_emit) {
         static_assert(12 * NT * sizeof(int32_t) >= 2 * NT * sizeof(int64_t), "scan table in the id table");
-        __shared__ int64_t wsa[NT / 64], wsb[NT / 64];
+        static_assert(256ll * kMcScanBlock * 64 * NZC * 5 < (1ll << 31), "mesh sizes in 32 bits");
+        __shared__ int wsa[NT / 64], wsb[NT / 64];
         int64_t *tab = reinterpret_cast<int64_t *>(&s.ids[0][0]);
         const int lane = tid & 63, wave = tid >> 6;
-        const int64_t a = tid < p.nblk ? (int64_t) p.bsum_v[tid] : 0, b = tid < p.nblk ? (int64_t) p.bsum_f[tid] : 0;
-        int64_t ia = a, ib = b;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int64_t ya = __shfl_up(ia, o), yb = __shfl_up(ib, o);
-            if (lane >= o) {
-                ia += ya;
-                ib += yb;
-            }
-        }
+        const int a = sum_v, b = sum_f, ia = wave_incl_sum(a), ib = wave_incl_sum(b);
         if (lane == 63) {
             wsa[wave] = ia;
             wsb[wave] = ib;
@@ -1187,12 +1181,13 @@ __device__ __forceinline__ void emit_tile(const McParams &p, int64_t tile, int s
             if (tid == 0) {
                 p.totals[0] = ta;
                 p.totals[1] = tb;
-                if (ta > 0x7fffffffll || tb > 0x7fffffffll) set_err(p, ISO_ERR_TOO_LARGE);
             }
         }
         __syncthreads();
         bv_tab = tab;
         bf_tab = tab + NT;
+    } else if (*(volatile int *) p.err & ISO_ERR_TOO_LARGE) {
+        return;
     }
 
     const int64_t tk = tile % p.NK, tj = (tile / p.NK) % p.NJ, ti = tile / (p.NK * p.NJ);
@@ -1645,27 +1640,37 @@ __device__ __forceinline__ void emit_tile(const McParams &p, int64_t tile, int s
 // built the list (blocks past the list's length have nothing to do), else b.
 __device__ __forceinline__ int64_t emit_block_tile(const McParams &p) {
     if (!p.tile_list) return blockIdx.x;
-    return (int) blockIdx.x < *p.tile_count ? (int64_t) p.tile_list[blockIdx.x] : -1;
+    const int t = p.tile_list[blockIdx.x];   // loaded beside the count: the list has room for every block
+    return (int) blockIdx.x < *p.tile_count ? (int64_t) t : -1;
 }
 
 // Five waves per SIMD: 96 VGPRs, and the narrow LDS slot types keep the
 // (16, 16, 2) and smaller tiles under 32 KB (five workgroups per CU).
 template <int TX, int TY, int NZC, int NT>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5, 8))) k_emit(McParams p) {
+    // one round of loads: the tile and the lane's block totals
+    const bool sums = p.scan_in_emit && (int) threadIdx.x < (int) p.nblk;
+    const int sv = sums ? (int) p.bsum_v[threadIdx.x] : 0, sf = sums ? (int) p.bsum_f[threadIdx.x] : 0;
     const int64_t tile = emit_block_tile(p);
-    if (tile >= 0) emit_tile<TX, TY, NZC, NT>(p, tile, (int) (blockIdx.x % p.seg.nseg));
+    if (tile >= 0) emit_tile<TX, TY, NZC, NT>(p, tile, (int) (blockIdx.x % p.seg.nseg), sv, sf);
 }
 
 template <int TX, int TY, int NZC, int NT>
 __global__ void __launch_bounds__(NT) k_emit_spheres(McParams p) {
+    // one round of loads: the tile and the lane's block totals
+    const bool sums = p.scan_in_emit && (int) threadIdx.x < (int) p.nblk;
+    const int sv = sums ? (int) p.bsum_v[threadIdx.x] : 0, sf = sums ? (int) p.bsum_f[threadIdx.x] : 0;
     const int64_t tile = emit_block_tile(p);
-    if (tile >= 0) emit_tile<TX, TY, NZC, NT, kSrcSpheres>(p, tile, (int) (blockIdx.x % p.seg.nseg));
+    if (tile >= 0) emit_tile<TX, TY, NZC, NT, kSrcSpheres>(p, tile, (int) (blockIdx.x % p.seg.nseg), sv, sf);
 }
 
 template <int TX, int TY, int NZC, int NT>
 __global__ void __launch_bounds__(NT) k_emit_program(McParams p) {
+    // one round of loads: the tile and the lane's block totals
+    const bool sums = p.scan_in_emit && (int) threadIdx.x < (int) p.nblk;
+    const int sv = sums ? (int) p.bsum_v[threadIdx.x] : 0, sf = sums ? (int) p.bsum_f[threadIdx.x] : 0;
     const int64_t tile = emit_block_tile(p);
-    if (tile >= 0) emit_tile<TX, TY, NZC, NT, kSrcProgram>(p, tile, (int) (blockIdx.x % p.seg.nseg));
+    if (tile >= 0) emit_tile<TX, TY, NZC, NT, kSrcProgram>(p, tile, (int) (blockIdx.x % p.seg.nseg), sv, sf);
 }
 
 // Reset of the per-call counters (and the active-tile flags when listed);
@@ -1679,6 +1684,20 @@ __global__ void mc_dense_reset(McParams p, SpecialLists init) {
 // Workgroup b copies segment b of every list; its offset is the sum of the
 // (clamped) counts of the segments before it.
 static_assert(kSpSeg == 256, "sp_gather_seg maps one thread to each segment");
+// The call's read-back, by one thread of the last kernel; dup is written by
+// the duplicate check.
+__device__ __forceinline__ void host_result(const McParams &p, const unsigned long long n[4], unsigned long long need) {
+    McHostResult *h = p.host;
+    h->err = *p.err;
+    h->totals[0] = p.totals[0];
+    h->totals[1] = p.totals[1];
+    h->sp.n_cand = n[0];
+    h->sp.n_scell = n[1];
+    h->sp.n_kept = n[2];
+    h->sp.n_hole = n[3];
+    h->sp.need = (int64_t) need;
+}
+
 __device__ __forceinline__ void sp_gather_seg(const McParams &p, int b) {
     // 256 threads, nseg <= 256: thread t reads segment t's four counters in
     // one round of loads; the offsets (clamped counts of the segments before
@@ -1746,6 +1765,7 @@ __device__ __forceinline__ void sp_gather_seg(const McParams &p, int b) {
         p.sp->n_kept = raw[2];
         p.sp->n_hole = raw[3];
         p.sp->need = (int64_t) nd;
+        if (p.host) host_result(p, raw, nd);
     }
 }
 
@@ -1776,15 +1796,23 @@ __device__ __forceinline__ void sp_dup_insert(const McParams &p, int32_t i) {
         const SpecialVertex o = cv[cur];
         if (o.x == v.x && o.y == v.y && o.z == v.z) {
             atomicExch((unsigned long long *) &p.sp->dup, 1ull);
+            if (p.host) p.host->sp.dup = 1;
             break;
         }
     }
 }
 
 // Workgroups [0, nseg) gather segment b of the special lists; the others
-// check the candidates for duplicate positions, segment by segment.
+// check the candidates for duplicate positions, segment by segment.  Without
+// a special entry (sp_any) the lists are as the reset left them: the launch
+// ends after one load (5 -> 2 us), and only the read-back is written.
 __global__ void __launch_bounds__(256) k_sp_gather_dup(McParams p) {
     const int nseg = p.seg.nseg;
+    if (p.sp_any && *p.sp_any == 0) {
+        const unsigned long long none[4] = {0, 0, 0, 0};
+        if (p.host && blockIdx.x == 0 && threadIdx.x == 0) host_result(p, none, 0);
+        return;
+    }
     if ((int) blockIdx.x < nseg) {
         sp_gather_seg(p, blockIdx.x);
         return;
