@@ -23,7 +23,8 @@ _by_shape: dict = {}   # shape -> configuration (cleared when the table changes)
 
 # (TX, TY, NZC) of each compiled configuration, in library order
 # (configuration 6 is the read-once pipeline: k_stream regions + 16 x 16 face tiles)
-CONFIGS = [(16, 16, 4), (8, 8, 2), (16, 16, 2), (16, 16, 1), (16, 16, 8), (8, 8, 1), (16, 16, 1)]
+CONFIGS = [(16, 16, 4), (8, 8, 2), (16, 16, 2), (16, 16, 1), (16, 16, 8), (8, 8, 1), (16, 16, 1),
+           (4, 4, 1)]
 
 
 def size_class(shape) -> str:

@@ -2274,7 +2274,8 @@ __global__ void k_its_reset(McParams p) {
     X(3, 16, 16, 1, 256)    \
     X(4, 16, 16, 8, 256)    \
     X(5, 8, 8, 1, 256)      \
-    X(6, 16, 16, 1, 256)
+    X(6, 16, 16, 1, 256)    \
+    X(7, 4, 4, 1, 256)
 
 int mc_config_count() {
     int n = 0;
@@ -2307,13 +2308,20 @@ int64_t mc_config_tiles(int cfg, const int64_t shape[3]) {
 }
 
 // First tile in the order that still gives every CU several workgroups
-// (16x16x64 cells from about 384^3 up, 8x8x128 near 256^3); when none
-// does, the one with the most tiles.  With empty tiles skipped through the
+// (16x16x64 cells from about 384^3 up, 8x8x64 near 256^3); when none does,
+// the one with the most tiles (4x4x64).  On a small grid the emit is one
+// round of workgroups and takes as long as its fullest tile: quarter tiles
+// halve the cells that one workgroup walks one batch after another (whole
+// call 8x8x64 -> 4x4x64: 64^3 49.0 -> 45.5 us, 128^3 62.3 -> 55.3, 192^3
+// with 1728 8x8x64 tiles 60.9 -> 58.5), while from 2048 tiles on the halo
+// read again by each tile costs more (224^3, 3136 tiles, 79.8 -> 88.3;
+// 256^3 125 -> 141).  128 threads a tile: 64^3 45.1, 160^3 61.9 instead of
+// 60.0; 64 threads 51.5 at 64^3.  With empty tiles skipped through the
 // active-tile list, 16x16x64 extracted fastest at 384^3..1024^3 on MI355X
 // (0.5-8% ahead of 16x16x128, which never has more tiles and so is not in
 // the order); 16x16x256 never wins.
 int mc_auto_config(const int64_t shape[3]) {
-    static const int order[] = {3, 1, 5};
+    static const int order[] = {3, 1, 5, 7};
     constexpr int64_t kWant = 2048;
     int best = 0;
     int64_t best_tiles = -1;
