@@ -244,15 +244,30 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // k_classify_v4 (Z % 64 == 0, float4-aligned rows): word w covers values
 // [64w, 64w + 64); 16 lanes load it with dwordx4 loads and merge their
 // nibbles with three in-group shuffles.
-// RESET: the grid first clears the extraction's state (reset_state), which
-// nothing in classify reads, so the stored-grid pipeline needs no separate
-// reset launch.
+// RESET: the grid's first kResetBlocks workgroups clear the extraction's
+// state (reset_state), which nothing in classify reads, so the stored-grid
+// pipeline needs no separate reset launch.
+// HBM-bound, and the mask writes between the reads cost more than their 3%
+// of the bytes: the same loop without them reads 4 GiB at 6.9 TB/s.  A wave
+// takes one step of kClassifyWords words and ends, so that the grid sweeps
+// the values in order; 8192 workgroups walking strided let the reads and
+// writes of 30 separate places interleave: 1024^3 772 -> 693 us (6.2 TB/s),
+// 509x387x451 (the flat kernel below) 64.8 -> 60.2 us.  8 words a step:
+// 683 us at 1024^3 but 14.6 instead of 13.6 us at 256^3; whole 128-byte
+// lines of masks, LDS-gathered masks and nontemporal mask stores changed
+// nothing.  The prologue is why only some workgroups reset: with all of
+// them 8 words a step took 732 us.
+constexpr int kClassifyWords = 16;               // per wave and step
+constexpr int64_t kClassifyBlocks = 1 << 23;     // 2^31 threads (a launch holds below 2^32); beyond: grid stride
+constexpr unsigned kResetBlocks = 1024;
 template <bool RESET>
 __global__ void __launch_bounds__(256) k_classify_v4(const float *__restrict__ values, int64_t nwords, float level,
                                                      uint64_t *__restrict__ bits, McParams rp, SpecialLists init) {
     if constexpr (RESET)
-        reset_state(rp, init, (int64_t) blockIdx.x * blockDim.x + threadIdx.x, (int64_t) gridDim.x * blockDim.x);
-    constexpr int U = 4;   // words in flight per 16-lane group
+        if (blockIdx.x < kResetBlocks)
+            reset_state(rp, init, (int64_t) blockIdx.x * 256 + threadIdx.x,
+                        (int64_t) min(gridDim.x, kResetBlocks) * 256);
+    constexpr int U = kClassifyWords / 4;   // words in flight per 16-lane group
     const int lane = threadIdx.x & 63;
     const int grp = lane >> 4, q = lane & 15;
     const int64_t wave = (int64_t) blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -338,7 +353,9 @@ __global__ void __launch_bounds__(256) k_classify(const float *__restrict__ valu
                                                   float level, uint64_t *__restrict__ bits, McParams rp,
                                                   SpecialLists init) {
     if constexpr (RESET)
-        reset_state(rp, init, (int64_t) blockIdx.x * blockDim.x + threadIdx.x, (int64_t) gridDim.x * blockDim.x);
+        if (blockIdx.x < kResetBlocks)
+            reset_state(rp, init, (int64_t) blockIdx.x * 256 + threadIdx.x,
+                        (int64_t) min(gridDim.x, kResetBlocks) * 256);
     __shared__ uint64_t ballots[4][kFlatChunks + 1];
     const int64_t wave = __builtin_amdgcn_readfirstlane((int) (blockIdx.x * 4 + (threadIdx.x >> 6)));
     const int64_t nwave = (int64_t) gridDim.x * 4;
@@ -1876,7 +1893,9 @@ __global__ void __launch_bounds__(256) k_classify_batch(const McBatchItem *__res
                                                         const McBatchHdr *__restrict__ hdr) {
     __shared__ int64_t starts[kMaxBatch];
     __shared__ uint64_t ballots[4][kFlatChunks + 1];
-    reset_batch_state(items, hdr, (int64_t) blockIdx.x * 256 + threadIdx.x, (int64_t) gridDim.x * 256);
+    if (blockIdx.x < kResetBlocks)
+        reset_batch_state(items, hdr, (int64_t) blockIdx.x * 256 + threadIdx.x,
+                          (int64_t) min(gridDim.x, kResetBlocks) * 256);
     const int n = (int) hdr->n;
     const int64_t ntask = hdr->nctask;
     for (int i = threadIdx.x; i < n; i += 256) starts[i] = items[i].ctask0;
@@ -2379,7 +2398,8 @@ static bool launch_classify(const McParams &p, hipStream_t stream, const Special
         const unsigned blocks = (unsigned) std::max<int64_t>(1, std::min<int64_t>((ntask + 3) / 4, 8192));
         hipLaunchKernelGGL(k_classify_spheres, dim3(blocks), dim3(256), 0, stream, p);
     } else if (p.vec4 && p.Z % 64 == 0) {
-        const unsigned blocks = (unsigned) std::max<int64_t>(1, std::min<int64_t>((nwords + 63) / 64, 8192));
+        const int64_t nb = (nwords + 4 * kClassifyWords - 1) / (4 * kClassifyWords);
+        const unsigned blocks = (unsigned) std::max<int64_t>(1, std::min(nb, kClassifyBlocks));
         if (reset)
             hipLaunchKernelGGL(k_classify_v4<true>, dim3(blocks), dim3(256), 0, stream, p.values, nwords, p.level,
                                p.bits, p, *reset);
@@ -2389,7 +2409,7 @@ static bool launch_classify(const McParams &p, hipStream_t stream, const Special
         return reset != nullptr;
     } else {
         const int64_t N = p.X * p.Y * p.Z, ntask = (N + kFlatPts - 1) / kFlatPts;
-        const unsigned blocks = (unsigned) std::max<int64_t>(1, std::min<int64_t>((ntask + 3) / 4, 8192));
+        const unsigned blocks = (unsigned) std::max<int64_t>(1, std::min<int64_t>((ntask + 3) / 4, kClassifyBlocks));
         if (reset)
             hipLaunchKernelGGL(k_classify<true>, dim3(blocks), dim3(256), 0, stream, p.values, N, p.Z, p.W, p.level,
                                p.bits, p, *reset);
@@ -2523,7 +2543,7 @@ hipError_t mc_batch_count_launch(const McBatchItem *items, const McBatchHdr *hdr
     hipError_t e = mc_upload_luts();
     if (e != hipSuccess) return e;
     // the classify kernel clears the batch's state first (no reset launch)
-    const unsigned cb = (unsigned) std::max<int64_t>(1, std::min<int64_t>((h.nctask + 3) / 4, 8192));
+    const unsigned cb = (unsigned) std::max<int64_t>(1, std::min<int64_t>((h.nctask + 3) / 4, kClassifyBlocks));
     hipLaunchKernelGGL(k_classify_batch, dim3(cb), dim3(256), 0, stream, items, hdr);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (h.ngtask > 0) {
