@@ -400,11 +400,94 @@ __device__ __forceinline__ int64_t entry_chunk(const McParams &p, int64_t i) {
     return r * p.W + s * p.nzc;
 }
 
+// Position of chunk g and the mask words its counts need: its own, the
+// rows' at x + 1 / y + 1, and the next word of each (0 where there is none).
+struct ChunkWords {
+    int64_t r, c, seg;
+    bool hasx, hasy, hxy;
+    uint64_t b, bn, bx, by, bxy, byn, bxn, bxyn;
+};
+
+__device__ __forceinline__ ChunkWords chunk_words(const McParams &p, int64_t g) {
+    ChunkWords k;
+    int64_t x, y;
+    if (p.narrow) {
+        const uint32_t g32 = (uint32_t) g, r32 = p.div_w.div(g32), c32 = g32 - r32 * (uint32_t) p.W,
+                       x32 = p.div_y.div(r32);
+        k.r = r32;
+        k.c = c32;
+        x = x32;
+        y = r32 - x32 * (uint32_t) p.Y;
+        k.seg = p.div_zc.div(c32);
+    } else {
+        k.r = div_fast(g, p.W);
+        k.c = g - k.r * p.W;
+        x = div_fast(k.r, p.Y);
+        y = k.r - x * p.Y;
+        k.seg = div_fast(k.c, p.nzc);
+    }
+    k.hasx = x + 1 < p.X;
+    k.hasy = y + 1 < p.Y;
+    k.hxy = k.hasx && k.hasy;
+    // all eight words are loaded before any is used: one memory round trip
+    // instead of two
+    const bool hn = k.c + 1 < p.W, hxyn = k.hxy && hn;
+    const int64_t YW = p.Y * p.W;
+    const uint64_t *q = p.bits + g;
+    k.b = q[0];
+    k.bn = hn ? q[1] : 0ull;
+    k.bx = k.hasx ? q[YW] : 0ull;
+    k.by = k.hasy ? q[p.W] : 0ull;
+    k.bxy = k.hxy ? q[YW + p.W] : 0ull;
+    k.byn = hxyn ? q[p.W + 1] : 0ull;
+    k.bxn = hxyn ? q[YW + 1] : 0ull;
+    k.bxyn = hxyn ? q[YW + p.W + 1] : 0ull;
+    return k;
+}
+
+// Whether chunk g may own a crossing edge or an active cell: not when its
+// word and those at x + 1, y + 1 and both are all clear, or all set, and so
+// are the points that follow.  The words at flat offsets past a row,
+// slab or grid end are not the chunk's neighbours; reading them anyway can
+// only call an empty chunk mixed, never the reverse, so no position is
+// needed.  Every lane of the wave calls it with consecutive g.
+__device__ __forceinline__ bool chunk_mixed(const McParams &p, int64_t g, int64_t total, bool inner) {
+    int64_t dy = p.W, dx = p.Y * p.W, dxy = dx + dy;
+    if (!inner) {   // a clamped offset is past every neighbour that exists
+        g = min(g, total - 1);
+        dy = min(dy, total - 1 - g);
+        dx = min(dx, total - 1 - g);
+        dxy = min(dxy, total - 1 - g);
+    }
+    const uint64_t *q = p.bits + g;
+    const uint64_t b = q[0], by = q[dy], bx = q[dx], bxy = q[dxy];
+    uint32_t last = 0;   // bit 0 of the next words, or-ed and and-ed: the next lane's, loaded by the last lane
+    if ((threadIdx.x & 63) == 63) {
+        const int64_t lim = total - 1 - g;
+        const uint64_t nb = q[min<int64_t>(1, lim)], ny = q[min(dy + 1, lim)], nx = q[min(dx + 1, lim)],
+                       nxy = q[min(dxy + 1, lim)];
+        last = (uint32_t) ((nb | ny | nx | nxy) & 1) | (uint32_t) (nb & ny & nx & nxy & 1) << 1;
+    }
+    const uint64_t any = b | by | bx | bxy, all = b & by & bx & bxy;
+    const uint32_t own = (uint32_t) (any & 1) | (uint32_t) (all & 1) << 1;
+    const uint32_t nxt =
+        (uint32_t) __builtin_amdgcn_update_dpp((int) last, (int) own, 0x130, 0xf, 0xf, false);   // wave_shl:1
+    return !((any == 0 && !(nxt & 1)) || (all == ~0ull && (nxt & 2)));
+}
+
 // One workgroup per kMcScanBlock entries.  Lanes walk the block's chunks in
 // memory order (coalesced mask loads), add their counts into the chunk's
 // entry in LDS, then the entries are scanned.  NT = 1024 for grids with few
 // blocks (more lanes in flight per block), 256 otherwise.
-template <int NT>
+// QUEUED: a wave first only looks for the chunks that a surface crosses and
+// queues them, and counts 64 queued ones at a time (their words come from
+// L1 or L2 again): the count is bound by VALU issue, and on a large grid
+// most chunks are empty (1024^3 162 -> 133 us, of which the masks' bytes
+// take 40; 509x387x451 28.6 -> 26.2).  Two or four chunks' words in flight
+// a lane: 136 and 144 us.  On few blocks the second trip for the words costs
+// more (64^3 8.9 -> 10.4 us), and so in intersection mode, where a chunk
+// counts in fewer instructions (batch of four to 430^3, 31.5 -> 35.2).
+template <int NT, bool QUEUED>
 __device__ __forceinline__ void count_block(const McParams &p, int64_t blk) {
     constexpr int PER = kMcScanBlock / NT;
     __shared__ uint32_t ent_v[kMcScanBlock], ent_f[kMcScanBlock];
@@ -425,49 +508,24 @@ __device__ __forceinline__ void count_block(const McParams &p, int64_t blk) {
     __syncthreads();
     const int64_t g0 = entry_chunk(p, i0);
     const int64_t g1 = i1 < n ? entry_chunk(p, i1) : p.X * p.Y * p.W;
-    const int64_t YW = p.Y * p.W;
     const int lane = tid & 63, wave = tid >> 6;
     __shared__ int32_t mark[NT / 64][64];
-    const bool narrow = p.narrow;
-    for (int64_t gb = g0; gb < g1; gb += NT) {   // every lane runs every round (wave-wide steps below)
-        const int64_t g = gb + tid;
-        const bool valid = g < g1;
-        const int64_t gg = valid ? g : g0;
-        int64_t r, c, x, y, seg;
-        if (narrow) {
-            const uint32_t g32 = (uint32_t) gg, r32 = p.div_w.div(g32), c32 = g32 - r32 * (uint32_t) p.W,
-                           x32 = p.div_y.div(r32);
-            r = r32;
-            c = c32;
-            x = x32;
-            y = r32 - x32 * (uint32_t) p.Y;
-            seg = p.div_zc.div(c32);
-        } else {
-            r = div_fast(gg, p.W);
-            c = gg - r * p.W;
-            x = div_fast(r, p.Y);
-            y = r - x * p.Y;
-            seg = div_fast(c, p.nzc);
-        }
-        const bool hasx = x + 1 < p.X, hasy = y + 1 < p.Y, hn = c + 1 < p.W;
-        const int64_t zlo = 64 * c;
-        // all eight words are loaded before any is used: one memory round
-        // trip per round instead of two
-        const bool hxy = hasx && hasy, hxyn = hxy && hn;
-        const uint64_t *q = p.bits + gg;
-        const uint64_t b = q[0], bn = hn ? q[1] : 0ull;
-        const uint64_t bx = hasx ? q[YW] : 0ull, by = hasy ? q[p.W] : 0ull;
-        const uint64_t bxy = hxy ? q[YW + p.W] : 0ull;
-        const uint64_t byn = hxyn ? q[p.W + 1] : 0ull, bxn = hxyn ? q[YW + 1] : 0ull,
-                       bxyn = hxyn ? q[YW + p.W + 1] : 0ull;
-        uint32_t cv = p.its ? 0u : (uint32_t) chunk_vertices(b, bn & 1, bx, by, hasx, hasy, zlo, p.Z);
+    // chunks found, relative to g0 (a block spans at most 8 * kMcScanBlock chunks)
+    __shared__ uint16_t queue[QUEUED ? NT / 64 : 1][128];
+    int queued = 0;
+    const int64_t total = p.X * p.Y * p.W;
+    const bool inner = g1 + NT + p.Y * p.W + p.W < total;   // no lane reads past the masks
+    // counts of one chunk a lane (valid: this lane has one)
+    auto count_chunks = [&](const ChunkWords &w, bool valid) {
+        const int64_t zlo = 64 * w.c;
+        uint32_t cv = p.its ? 0u : (uint32_t) chunk_vertices(w.b, w.bn & 1, w.bx, w.by, w.hasx, w.hasy, zlo, p.Z);
         uint32_t cf = 0;
-        const CellMasks m = cell_masks(b, bn, by, byn, bx, bxn, bxy, bxyn);
-        uint64_t act = hxy ? cell_active(m) & low_bits(p.Z - 1 - zlo) : 0ull;
+        const CellMasks m = cell_masks(w.b, w.bn, w.by, w.byn, w.bx, w.bxn, w.bxy, w.bxyn);
+        uint64_t act = w.hxy ? cell_active(m) & low_bits(p.Z - 1 - zlo) : 0ull;
         // bit 0 of the next word of rows (0,0), (0,1), (1,0), (1,1)
-        const uint32_t nxt = (uint32_t) (bn & 1) | (uint32_t) (byn & 1) << 1 | (uint32_t) (bxn & 1) << 2 |
-                             (uint32_t) (bxyn & 1) << 3;
-        if (hxy) {
+        const uint32_t nxt = (uint32_t) (w.bn & 1) | (uint32_t) (w.byn & 1) << 1 | (uint32_t) (w.bxn & 1) << 2 |
+                             (uint32_t) (w.bxyn & 1) << 3;
+        if (w.hxy) {
             if (p.its) {
                 // crossing edges of the active cells, bit-parallel over the 64
                 // cells: edge e crosses where its two corner masks differ
@@ -476,10 +534,10 @@ __device__ __forceinline__ void count_block(const McParams &p, int64_t blk) {
             }
         }
         if (!valid) act = 0;
-        const int e = (int) (r * p.S + seg - i0);
+        const int e = (int) (w.r * p.S + w.seg - i0);
         if (valid && cv) atomicAdd(&ent_v[e], cv);
         if (valid && cf) atomicAdd(&ent_f[e], cf);
-        if (p.its) continue;
+        if (p.its) return;
         // triangles: the wave's active cells are dealt out one per lane per
         // round (owner lane by a running maximum over marked first slots),
         // so a word with many active cells does not serialise its wave
@@ -494,7 +552,7 @@ __device__ __forceinline__ void count_block(const McParams &p, int64_t blk) {
             const int own = max(wave_incl_max(mark[wave][lane]), 0);
             const int k = base + lane;
             const uint64_t oact = __shfl(act, own);
-            const uint64_t w00 = __shfl(b, own), w01 = __shfl(by, own), w10 = __shfl(bx, own), w11 = __shfl(bxy, own);
+            const uint64_t w00 = __shfl(w.b, own), w01 = __shfl(w.by, own), w10 = __shfl(w.bx, own), w11 = __shfl(w.bxy, own);
             const uint32_t on = (uint32_t) __shfl((int) nxt, own);
             const int oexcl = __shfl(excl, own), oe = __shfl(e, own);
             if (k < total) {
@@ -511,6 +569,31 @@ __device__ __forceinline__ void count_block(const McParams &p, int64_t blk) {
                 atomicAdd(&ent_f[oe], (uint32_t) ntri[cs]);
             }
             __builtin_amdgcn_wave_barrier();
+        }
+    };
+    for (int64_t gb = g0; gb < g1 || queued > 0;) {   // every lane runs every round (wave-wide steps)
+        if constexpr (QUEUED) {
+            while (gb < g1 && queued < 64) {
+                const int64_t g = gb + tid;
+                const bool hit = chunk_mixed(p, g, total, inner) && g < g1;
+                const uint64_t hits = __ballot(hit);
+                if (hit) queue[wave][queued + __popcll(hits & ((1ull << lane) - 1))] = (uint16_t) (g - g0);
+                queued += __popcll(hits);
+                gb += NT;
+            }
+            __builtin_amdgcn_wave_barrier();
+            const int take = min(queued, 64);
+            if (take > 0) {
+                // from the end: what is left stays in place
+                const int64_t g = g0 + queue[wave][queued - take + (lane < take ? lane : 0)];
+                __builtin_amdgcn_wave_barrier();
+                queued -= take;
+                count_chunks(chunk_words(p, g), lane < take);
+            }
+        } else {
+            const int64_t g = gb + tid;
+            count_chunks(chunk_words(p, g < g1 ? g : g0), g < g1);
+            gb += NT;
         }
     }
     __syncthreads();
@@ -550,11 +633,12 @@ __device__ __forceinline__ void count_block(const McParams &p, int64_t blk) {
     }
 }
 
-template <int NT>
-__global__ void __launch_bounds__(NT) k_count(McParams p) { count_block<NT>(p, blockIdx.x); }
+template <int NT, bool QUEUED>
+__global__ void __launch_bounds__(NT) k_count(McParams p) { count_block<NT, QUEUED>(p, blockIdx.x); }
 
-// Blocks below which the count pass uses 1024-lane workgroups.
-constexpr int64_t kCountWideBelow = 2048;
+// Blocks below which the count pass uses 1024-lane workgroups, and from
+// which those queue the chunks that the surface crosses.
+constexpr int64_t kCountWideBelow = 2048, kCountQueuedFrom = 512;
 
 // Exclusive scan of the block totals by one workgroup: thread t sums a
 // contiguous run of ceil(nblk / 1024) totals, one block-wide scan of the run
@@ -2003,7 +2087,7 @@ __global__ void __launch_bounds__(NT) k_count_batch(const McBatchItem *__restric
     for (int i = threadIdx.x; i < n; i += NT) starts[i] = items[i].blk0;
     __syncthreads();
     const int i = __builtin_amdgcn_readfirstlane(find_start(starts, n, gb));
-    count_block<NT>(items[i].p, gb - items[i].blk0);
+    count_block<NT, NT == 256>(items[i].p, gb - items[i].blk0);
 }
 
 __global__ void __launch_bounds__(1024) k_scan_top_batch(const McBatchItem *__restrict__ items,
@@ -2421,6 +2505,16 @@ static bool launch_classify(const McParams &p, hipStream_t stream, const Special
     return false;
 }
 
+static void launch_count(const McParams &p, hipStream_t stream) {
+    const dim3 blocks((unsigned) p.nblk);
+    if (p.nblk >= kCountWideBelow)
+        hipLaunchKernelGGL((k_count<256, true>), blocks, dim3(256), 0, stream, p);
+    else if (p.nblk >= kCountQueuedFrom && !p.its)
+        hipLaunchKernelGGL((k_count<1024, true>), blocks, dim3(1024), 0, stream, p);
+    else
+        hipLaunchKernelGGL((k_count<1024, false>), blocks, dim3(1024), 0, stream, p);
+}
+
 void mc_params_divisors(McParams &p) {
     p.narrow = p.X > 0 && p.Y > 0 && p.W > 0 && p.nzc > 0 && p.X * p.Y * p.W <= (int64_t) UINT32_MAX;
     if (p.narrow) {
@@ -2461,10 +2555,7 @@ hipError_t mc_dense_launch(int cfg, McParams &p, const SpecialLists &sp_init, hi
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if ((e = mark(1)) != hipSuccess) return e;
 
-    if (p.nblk < kCountWideBelow)
-        hipLaunchKernelGGL(k_count<1024>, dim3((unsigned) p.nblk), dim3(1024), 0, stream, p);
-    else
-        hipLaunchKernelGGL(k_count<256>, dim3((unsigned) p.nblk), dim3(256), 0, stream, p);
+    launch_count(p, stream);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if ((e = mark(2)) != hipSuccess) return e;
     // up to 256 count blocks the emit workgroups scan the block totals
@@ -2514,10 +2605,7 @@ hipError_t its_dense_count_launch(McParams &p, hipStream_t stream) {
     }
     const SpecialLists none{};
     launch_classify(p, stream, grid_field ? &none : nullptr);
-    if (p.nblk < kCountWideBelow)
-        hipLaunchKernelGGL(k_count<1024>, dim3((unsigned) p.nblk), dim3(1024), 0, stream, p);
-    else
-        hipLaunchKernelGGL(k_count<256>, dim3((unsigned) p.nblk), dim3(256), 0, stream, p);
+    launch_count(p, stream);
     hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, stream, p);
     return hipGetLastError();
 }
