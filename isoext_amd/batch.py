@@ -101,23 +101,19 @@ def _items(jobs, who):
     dev = jobs[0].device
     items = (McItem * len(jobs))()
     for it, j in zip(items, jobs):
+        t = j.values
         if j.sdf is not None:
             if j.sdf.device != dev or j.shape is None or len(j.shape) != 3:
                 raise TypeError(f"{who}: an SDF job needs a program on the batch's device and a 3-entry shape")
-            it.values = None
             it.sdf = j.sdf.ptr
             it.sdf_normals = 1 if j.sdf_normals else 0
         else:
-            if j.values.device != dev or j.values.dtype != torch.float32 or not j.values.is_contiguous():
+            if t.device != dev or t.dtype != torch.float32 or not t.is_contiguous():
                 raise TypeError(f"{who}: values must be contiguous float32 tensors on one device")
-            it.values = j.values.data_ptr()
-            it.sdf = None
-            it.sdf_normals = 0
-        shape = j.grid_shape
-        for a in range(3):
-            it.shape[a] = shape[a]
-            it.aabb_min[a] = float(j.aabb_min[a])
-            it.aabb_max[a] = float(j.aabb_max[a])
+            it.values = t.data_ptr()
+        it.shape[:] = j.grid_shape[:3]
+        it.aabb_min[:] = [float(a) for a in j.aabb_min[:3]]
+        it.aabb_max[:] = [float(a) for a in j.aabb_max[:3]]
         it.level = float(j.level)
         it.method = int(j.method)
     return dev, items
@@ -214,32 +210,34 @@ def mc_batch(jobs: list[GridJob], cfg: int | None = BATCH_CFG, ws_kind: str = "m
         _lib.check(L.isoext_mc_batch_count(n, items, cfg, ws.data_ptr(), ws.numel(), special, counts, stream),
                    "mc_batch count")
         # one vertex and one face buffer for the batch; each grid gets a slice
-        nvs = [int(counts[2 * i]) for i in range(n)]
-        nfs = [int(counts[2 * i + 1]) for i in range(n)]
+        nvs, nfs = counts[0::2], counts[1::2]
         if on_sizes is not None:
             on_sizes([12 * a + 12 * b for a, b in zip(nvs, nfs)])
         all_v = torch.empty((max(sum(nvs), 1), 3), dtype=torch.float32, device=dev)
         all_f = torch.empty((max(sum(nfs), 1), 3), dtype=torch.int32, device=dev)
-        v0 = f0 = 0
-        outs = []
-        for i, it in enumerate(items):
-            it.out_v, it.cap_v = all_v.data_ptr() + 12 * v0, nvs[i]
-            it.out_f, it.cap_f = all_f.data_ptr() + 12 * f0, nfs[i]
-            outs.append((v0, f0))
-            v0 += nvs[i]
-            f0 += nfs[i]
+        pv, pf = all_v.data_ptr(), all_f.data_ptr()
+        for it, a, b in zip(items, nvs, nfs):
+            it.out_v, it.cap_v, it.out_f, it.cap_f = pv, a, pf, b
+            pv += 12 * a
+            pf += 12 * b
         rc = L.isoext_mc_batch_emit(n, items, cfg, ws.data_ptr(), ws.numel(), special, counts, stream)
     _lib.check(rc, "mc_batch emit")
     res = []
-    for i, (v0, f0) in enumerate(outs):
-        nv, nf = int(counts[2 * i]), int(counts[2 * i + 1])
-        v, f = all_v[v0:v0 + nvs[i]], all_f[f0:f0 + nfs[i]]
+    vs, fs = _pieces(all_v, counts[0::2], nvs), _pieces(all_f, counts[1::2], nfs)
+    for j, v, f, nv in zip(jobs, vs, fs, counts[0::2]):
         if nv < 0:   # special lists overflowed the batch capacity: run this grid alone
             from .mc import mc_dense_raw
-            j = jobs[i]
             v, f, _ = mc_dense_raw(j.values, j.grid_shape, j.aabb_min, j.aabb_max, j.level, j.method,
                                    cfg if cfg >= 0 else None, program=j.sdf)
-            res.append((v, f))
-        else:
-            res.append((v[:nv], f[:nf]))
+        res.append((v, f))
     return res
+
+
+def _pieces(buf, used, room):
+    """The first used[i] rows of each room[i] rows of buf (none if used[i] is
+    negative), as views from one call."""
+    sizes = []
+    for u, r in zip(used, room):
+        u = max(u, 0)
+        sizes += (u, r - u)
+    return buf.split([*sizes, buf.shape[0] - sum(room)])[:-1:2]

