@@ -227,7 +227,7 @@ struct McBatchHdr {
 };
 constexpr int kMaxTileConfigs = 8;
 
-// Per-item result of a batch phase, gathered for one read-back.
+// Per-item result of a batch phase, written to the host's pinned staging.
 struct McBatchSummary {
     int64_t err, nv, nf;
     SpecialLists sp;   // the item's contiguous special lists (counts, need)

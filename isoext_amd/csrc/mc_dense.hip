@@ -2380,6 +2380,10 @@ __global__ void k_its_reset(McParams p) {
     X(6, 16, 16, 1, 256)    \
     X(7, 4, 4, 1, 256)
 
+#define X(...) +1
+static_assert(0 ISO_MC_CONFIGS(X) <= kMaxTileConfigs, "a list length per tile configuration");
+#undef X
+
 int mc_config_count() {
     int n = 0;
 #define X(id, tx, ty, nzc, nt) ++n;
