@@ -344,10 +344,11 @@ __device__ __forceinline__ void jacobi_sym3(const T a[3][3], T w[3], T v[3][3], 
         for (int j = 0; j < 3; ++j) v[i][j] = (i == j) ? T(1) : T(0);
     for (int sw = 0; sw < sweeps; ++sw) {
         // done when what is left could not change a digit: a rotation turns by
-        // about off / gap, and moves an eigenvalue by its square over the gap
-        const T off = o[0] * o[0] + o[1] * o[1] + o[2] * o[2];
-        const T tr = fabs(d[0]) + fabs(d[1]) + fabs(d[2]);
-        if (off <= (sizeof(T) == 8 ? T(1e-40) : T(1e-20)) * tr * tr) break;   // NaN goes on
+        // about off / gap, and moves an eigenvalue by its square over the gap.
+        // Entries are compared as they are: their squares would overflow (or
+        // vanish) for normals far from unit length.  NaN and infinity go on.
+        const T tr = fabs(d[0]) + fabs(d[1]) + fabs(d[2]), lim = (sizeof(T) == 8 ? T(1e-20) : T(1e-10)) * tr;
+        if (fabs(o[0]) <= lim && fabs(o[1]) <= lim && fabs(o[2]) <= lim && tr < T(INFINITY)) break;
 #pragma unroll
         for (int r = 2; r >= 0; --r) {   // rotate the plane (p, q) without r
             const int p = r == 0 ? 1 : 0, q = r == 2 ? 1 : 2;
