@@ -213,22 +213,40 @@ _dc_hint: dict = {}
 _hint_lock = threading.Lock()
 
 
+# Most cells that a call without a hint makes room for; a call that needs more
+# is repeated with the counted size.
+_FIRST_CELLS = 1 << 22
+
+
+def _most_cells(shape):
+    n = 1
+    for s in shape:
+        n *= max(int(s) - 1, 0)
+    return max(n, 1)
+
+
+def _first_cells(shape):
+    # surface-like: a few times the largest cross-section
+    X, Y, Z = shape
+    return min(max(1 << 15, 2 * max(X * Y, Y * Z, X * Z)), _FIRST_CELLS, _most_cells(shape))
+
+
 def _its_caps(shape):
+    most = min(_most_cells(shape), 0x7fffffff)
     hint = _its_hint.get(shape)   # a single dict read needs no lock
     if hint is None:
-        # surface-like: a few times the largest cross-section
-        X, Y, Z = shape
-        cells = min(max(1 << 15, 2 * max(X * Y, Y * Z, X * Z)), 0x3fffffff)
+        cells = _first_cells(shape)
         return cells, 4 * cells
-    return hint[0] + hint[0] // 8 + 1024, hint[1] + hint[1] // 8 + 4096
+    return min(hint[0] + hint[0] // 8 + 1024, most), min(hint[1] + hint[1] // 8 + 4096, 12 * most)
 
 
 def _dc_caps(shape):
     hint = _dc_hint.get(shape)
     if hint is None:
-        nc = _its_caps(shape)[0]
+        nc = _first_cells(shape)
         return nc, nc, 2 * nc
-    return tuple(min(n + n // 8 + 1024, m) for n, m in zip(hint, (0x3fffffff, 1 << 31, 1 << 32)))
+    most = min(_most_cells(shape), 0x3fffffff)
+    return tuple(min(n + n // 8 + 1024, k * most) for n, k in zip(hint, (1, 1, 6)))
 
 
 def _its_buffers(nc, npt, normals, dev):

@@ -1,0 +1,36 @@
+"""Room that intersections and dual contouring of a dense grid start with:
+never more than the grid can hold, however flat it is, and no more than a
+few million cells on a guess."""
+
+import pytest
+
+from isoext_amd import dc
+
+
+def cells(shape):
+    return (shape[0] - 1) * (shape[1] - 1) * (shape[2] - 1)
+
+
+# flat grids have fewer cells than twice their cross-section; the last would pass 2^30 cells
+FLAT = [(2, 20000, 20000), (23200, 2, 23200), (30000, 30000, 2), (2, 2, 2), (2, 3, 64), (5, 5, 5), (40000, 40000, 2)]
+
+
+@pytest.mark.parametrize("shape", FLAT + [(1024, 1024, 1024), (1, 7, 9)])
+def test_first_room(monkeypatch, shape):
+    monkeypatch.setattr(dc, "_its_hint", {})
+    monkeypatch.setattr(dc, "_dc_hint", {})
+    most = max(cells(shape), 1)
+    nc, npt = dc._its_caps(shape)
+    assert 1 <= nc <= min(most, 1 << 22) and nc <= npt <= 12 * most
+    nc, cap_v, cap_f = dc._dc_caps(shape)
+    assert 1 <= nc <= min(most, 1 << 22) and cap_v <= nc and cap_f <= 2 * nc
+
+
+@pytest.mark.parametrize("shape", FLAT)
+def test_room_after_a_full_grid(monkeypatch, shape):
+    most = cells(shape)
+    monkeypatch.setattr(dc, "_its_hint", {shape: (most, 12 * most)})
+    monkeypatch.setattr(dc, "_dc_hint", {shape: (most, most, 6 * most)})
+    assert dc._its_caps(shape) == (most, 12 * most)
+    lim = min(most, 0x3fffffff)   # isoext_dc_grid's own limit
+    assert dc._dc_caps(shape) == (lim, lim, 6 * lim)
