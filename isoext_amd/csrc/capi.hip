@@ -318,9 +318,12 @@ struct DcLayout {
     size_t o_dual, o_cond, o_used, o_bnd, o_qn, o_qm, o_bsum, o_part, o_tot, o_tri, o_hs, o_rep, o_fin, o_ak, o_av,
         total;
     int64_t hslots;
+    bool hash;
 };
 
-DcLayout dc_layout(int64_t ncells, int64_t npts) {
+// hash: with the active-cell hash (24 to 48 B a cell), which a run on lookup
+// tables does without.
+DcLayout dc_layout(int64_t ncells, int64_t npts, bool hash = true) {
     DcLayout L;
     int64_t nb = (std::max(ncells, npts) + 255) / 256 + 1;
     int64_t hs = 1;
@@ -345,8 +348,9 @@ DcLayout dc_layout(int64_t ncells, int64_t npts) {
     L.o_hs = take(sizeof(int32_t) * hs);
     L.o_rep = take(sizeof(int32_t) * std::max<int64_t>(ncells, 1));
     L.o_fin = take(sizeof(int32_t) * std::max<int64_t>(ncells, 1));
-    L.o_ak = take(sizeof(int64_t) * hs);
-    L.o_av = take(sizeof(int32_t) * hs);
+    L.o_ak = hash ? take(sizeof(int64_t) * hs) : 0;
+    L.o_av = hash ? take(sizeof(int32_t) * hs) : 0;
+    L.hash = hash;
     L.total = o;
     return L;
 }
@@ -367,8 +371,8 @@ iso::DcScratch dc_scratch(char *ws, const DcLayout &L) {
     w.cap_tri = 6;
     w.hslots = (uint32_t *) (ws + L.o_hs);
     w.hmask = L.hslots - 1;
-    w.akey = (int64_t *) (ws + L.o_ak);
-    w.aval = (int32_t *) (ws + L.o_av);
+    w.akey = L.hash ? (int64_t *) (ws + L.o_ak) : nullptr;
+    w.aval = L.hash ? (int32_t *) (ws + L.o_av) : nullptr;
     w.amask = L.hslots - 1;
     w.rep_slot = (int32_t *) (ws + L.o_rep);
     w.final_id = (int32_t *) (ws + L.o_fin);
@@ -717,7 +721,7 @@ DcBatchLayout dc_batch_layout(int n, const isoext_mc_item *items, int64_t C, int
     L.o_qb = L.o_vb + sizeof(int64_t) * (size_t) (n + 1);
     L.o_tm = take(sizeof(uint64_t) * (size_t) std::max<int64_t>(T, 1));
     L.o_tp = take(sizeof(int32_t) * (size_t) std::max<int64_t>(T, 1));
-    L.dc = dc_layout(C, 0);
+    L.dc = dc_layout(C, 0, false);
     L.o_dc = take(L.dc.total);
     L.total = o;
     return L;
@@ -880,7 +884,7 @@ struct DcGridLayout {
         o_cd = take(sizeof(int64_t) * (size_t) cap_cells);
         o_tm = take(sizeof(uint64_t) * (size_t) T);
         o_tp = take(sizeof(int32_t) * (size_t) T);
-        dc = dc_layout(cap_cells, 0);
+        dc = dc_layout(cap_cells, 0, false);
         o_dc = take(dc.total);
         total = o;
     }

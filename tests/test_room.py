@@ -34,3 +34,18 @@ def test_room_after_a_full_grid(monkeypatch, shape):
     assert dc._its_caps(shape) == (most, 12 * most)
     lim = min(most, 0x3fffffff)   # isoext_dc_grid's own limit
     assert dc._dc_caps(shape) == (lim, lim, 6 * lim)
+
+
+def test_grid_workspace_per_cell():
+    """Lookup tables stand in for the active-cell hash: a cell takes its vertex, flags, ids and place in the scan
+    (about 40 B) and two to four position slots of 4 B, not another 24 to 48 B of hash."""
+    import ctypes
+
+    from isoext_amd import _lib
+    g = dc.IsoGrid()
+    g.values = 64   # any address: sizes only
+    for a in range(3):
+        g.shape[a], g.aabb_min[a], g.aabb_max[a] = 1024, -1.0, 1.0
+    size = _lib.lib().isoext_dc_grid_workspace_bytes
+    n = 1 << 20
+    assert (size(ctypes.byref(g), 2 * n) - size(ctypes.byref(g), n)) / n < 60
