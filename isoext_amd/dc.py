@@ -162,13 +162,15 @@ def get_intersection(grid, level: float = 0.0, compute_normals: bool = False) ->
     tables = None
     with torch.cuda.device(dev):
         stream = _lib.stream_ptr(dev)
-        if getattr(grid, "cell_ids", None) is None:
-            # dense: the buffers, sized by the last set of this shape, are made while the count runs, and only the
-            # counts are waited for
+        shape = tuple(g.shape)
+        dense = getattr(grid, "cell_ids", None) is None
+        if dense:
+            nt = max(int(L.isoext_its_table_entries(g.shape)), 1)
+        if dense and not _its_vary(shape):
+            # the buffers, sized by recent sets of this shape, are made while the count runs, and only the counts are
+            # waited for
             _lib.check(L.isoext_its_begin(ctypes.byref(g), float(level), scratch.data_ptr(), scratch.numel(), stream),
                        "get_intersection")
-            shape = tuple(g.shape)
-            nt = max(int(L.isoext_its_table_entries(g.shape)), 1)
             tables = (torch.empty(nt, dtype=torch.int64, device=dev), torch.empty(nt, dtype=torch.int32, device=dev))
             nc, npt = _its_caps(shape)
             for _ in range(2):
@@ -181,16 +183,11 @@ def get_intersection(grid, level: float = 0.0, compute_normals: bool = False) ->
                 nc, npt = int(counts[0]), int(counts[1])
             _lib.check(rc, "get_intersection")
             cap, nc, npt = npt, int(counts[0]), int(counts[1])
-            with _hint_lock:
-                if len(_its_hint) > 4096:
-                    _its_hint.clear()
-                _its_hint[shape] = (nc, npt)
             ends = (nc, nc, nc + 1, npt, npt, npt, npt, npt)
             b = [t[:n] if t is not None else None for t, n in zip(b, ends)]
-            if cap > 2 * npt + 65536:   # do not pin much larger buffers behind a small set
+            if cap > 2 * npt + _PINNED:   # do not pin much larger buffers behind a small set
                 b = [t.clone() if t is not None else None for t in b]
-            tables = tables if nc else None
-        elif g.n_sparse == 0:
+        elif not dense and g.n_sparse == 0:
             b = _its_buffers(0, 0, compute_normals, dev)
             b[2].zero_()
         else:
@@ -198,19 +195,54 @@ def get_intersection(grid, level: float = 0.0, compute_normals: bool = False) ->
                                           stream), "get_intersection")
             nc, npt = int(counts[0]), int(counts[1])
             b = _its_buffers(nc, npt, compute_normals, dev)
+            if dense:
+                tables = (torch.empty(nt, dtype=torch.int64, device=dev),
+                          torch.empty(nt, dtype=torch.int32, device=dev))
             p = [t.data_ptr() if t is not None and (npt or k < 3) else None for k, t in enumerate(b)]
-            _lib.check(L.isoext_its_emit(ctypes.byref(g), float(level), scratch.data_ptr(), nc, npt, *p, None, None,
+            _lib.check(L.isoext_its_emit(ctypes.byref(g), float(level), scratch.data_ptr(), nc, npt, *p,
+                                         *(t.data_ptr() for t in tables or ()), *(() if dense else (None, None)),
                                          stream), "get_intersection")
+        if dense:
+            _remember(_its_hint, shape, (nc, npt), _its_low)
+            tables = tables if nc else None
     cell_indices, cell_dense, cell_offsets, points, normals, edge_local, is_out, entry_cell = b
     return Intersection(grid, level, cell_indices, cell_dense, cell_offsets, points, normals, edge_local, is_out,
                         entry_cell, tables)
 
 
-# cells and points of the last intersection set of a dense shape, and cells and
-# faces of its last dual mesh (sizing hints)
+# cells and points of a dense shape's recent intersection sets, and cells,
+# vertices and faces of its recent dual meshes (sizing hints); points of its
+# recent small intersection sets
 _its_hint: dict = {}
 _dc_hint: dict = {}
+_its_low: dict = {}
 _hint_lock = threading.Lock()
+_PINNED = 65536   # entries that may be kept behind a smaller set, beyond its own size
+
+
+def _remember(hints, shape, sizes, low=None):
+    """The sizes of a call, or what is left of larger ones before it: those
+    fall by a 32nd a call.  With the eighth more that the next call makes room
+    for, a large surface still fits after three small ones of its shape (too
+    little room costs a second run), and a lone large one is soon forgotten.
+    low: the same of the last size from the other side."""
+    with _hint_lock:
+        if len(hints) > 4096:
+            hints.clear()
+        hints[shape] = tuple(max(n, o - o // 32) for n, o in zip(sizes, hints.get(shape, sizes)))
+        if low is not None:
+            if len(low) > 4096:
+                low.clear()
+            o = low.get(shape, sizes[-1])
+            low[shape] = min(sizes[-1], o + o // 32 + 32)
+
+
+def _its_vary(shape):
+    """Whether a shape's recent intersection sets differ so much that room for
+    the largest would mean copying the others out of it (eight copies, 40 us,
+    where waiting for the count before the buffers are made takes 20)."""
+    low = _its_low.get(shape)
+    return low is not None and shape in _its_hint and _its_caps(shape)[1] > 2 * low + _PINNED
 
 
 # Most cells that a call without a hint makes room for; a call that needs more
@@ -334,7 +366,7 @@ def dual_contouring(grid, level: float = 0.0, intersection: Intersection | None 
 
 def _dc_grid(grid, level: float, reg: float, svd_tol: float):
     """dual_contouring of a dense grid without an intersection set, into
-    buffers sized by the last mesh of this shape (one synchronisation)."""
+    buffers sized by recent meshes of this shape (one synchronisation)."""
     check_cuda_f32(grid.values, 3, name="values")
     dev = _device(grid)
     L = _lib.lib()
@@ -359,10 +391,7 @@ def _dc_grid(grid, level: float, reg: float, svd_tol: float):
                 cap_v, cap_f = max(cap_v, int(counts[0])), max(cap_f, int(counts[1]))
     _lib.check(rc, "dual_contouring")
     nv, nf = int(counts[0]), int(counts[1])
-    with _hint_lock:
-        if len(_dc_hint) > 4096:
-            _dc_hint.clear()
-        _dc_hint[shape] = (int(counts[3]), nv, nf)
+    _remember(_dc_hint, shape, (int(counts[3]), nv, nf))
     if nf == 0:
         return None, None
     v, f = out_v[:nv], out_f[:nf]

@@ -96,3 +96,29 @@ def test_refusals_and_empty(gpu):
     assert len(its) == 0 and its.cell_offsets.tolist() == [0]
     assert iso.dual_contouring(s) == (None, None)
     torch.cuda.synchronize()
+
+
+def test_small_and_large_surfaces_in_turn(gpu, monkeypatch):
+    """Each is run once: the room for the large one is kept over small ones between."""
+    import torch
+
+    import isoext_amd as iso
+    from isoext_amd import dc
+    shape = (60, 61, 62)
+    large = iso.UniformGrid.wrap(torch.from_numpy(field("noise", shape)).cuda())
+    small = iso.UniformGrid.wrap(torch.from_numpy(field("spheres", shape)).cuda())
+    runs = []
+    buffers, get = dc._its_buffers, dc.workspace.get
+    monkeypatch.setattr(dc, "_its_buffers", lambda *a: (runs.append("its"), buffers(*a))[1])
+    monkeypatch.setattr(dc.workspace, "get", lambda kind, *a: (runs.append(kind), get(kind, *a))[1])
+    monkeypatch.setattr(dc, "_its_hint", {})
+    monkeypatch.setattr(dc, "_dc_hint", {})
+    for g in (large, small, small, small, large, small, large):
+        a, b = (dc._its_hint.get(shape), dc._dc_hint.get(shape))
+        runs.clear()
+        its, mesh = iso.get_intersection(g, 0.0, True), iso.dual_contouring(g, 0.0)
+        if a is not None and b is not None:   # the first call knows nothing
+            assert runs.count("dc_grid") == 1 and runs.count("its") == 2   # scratch and one set of buffers
+        ref = counted(g, 0.0, True)
+        assert torch.equal(its.points, ref.points) and torch.equal(its.cell_offsets, ref.cell_offsets)
+        assert torch.equal(mesh[0], dc.dc_raw(g, ref, ref.normals, 1e-2, 1e-6)[0])
