@@ -122,3 +122,23 @@ def test_small_and_large_surfaces_in_turn(gpu, monkeypatch):
         ref = counted(g, 0.0, True)
         assert torch.equal(its.points, ref.points) and torch.equal(its.cell_offsets, ref.cell_offsets)
         assert torch.equal(mesh[0], dc.dc_raw(g, ref, ref.normals, 1e-2, 1e-6)[0])
+
+
+def test_grids_without_a_cell_in_turn(gpu, monkeypatch):
+    """After a grid without a cell the next of its shape is counted first."""
+    import torch
+
+    import isoext_amd as iso
+    from isoext_amd import dc
+    shape = (20, 21, 66)
+    none, some = (iso.UniformGrid.wrap(torch.from_numpy(field(k, shape)).cuda()) for k in ("none", "spheres"))
+    v, f = iso.dual_contouring(some, 0.03)
+    runs, caps = [], dc._dc_caps
+    monkeypatch.setattr(dc, "_dc_caps", lambda s: (runs.append(s), caps(s))[1])
+    monkeypatch.setattr(dc, "_dc_hint", {})
+    monkeypatch.setattr(dc, "_dc_none", set())
+    for g, run in ((none, 1), (none, 0), (none, 0), (some, 1), (some, 1), (none, 1), (none, 0), (some, 1)):
+        runs.clear()
+        a, b = iso.dual_contouring(g, 0.03)
+        assert len(runs) == run
+        assert a is None and b is None if g is none else torch.equal(a, v) and torch.equal(b, f)
