@@ -235,9 +235,10 @@ def mc_batch(jobs: list[GridJob], cfg: int | None = BATCH_CFG, ws_kind: str = "m
 
 def _pieces(buf, used, room):
     """The first used[i] rows of each room[i] rows of buf (none if used[i] is
-    negative), as views from one call."""
+    negative), from one call.  The unsafe split: autograd lets its pieces be
+    changed in place, and they never share a row."""
     sizes = []
     for u, r in zip(used, room):
         u = max(u, 0)
         sizes += (u, r - u)
-    return buf.split([*sizes, buf.shape[0] - sum(room)])[:-1:2]
+    return buf.unsafe_split_with_sizes([*sizes, buf.shape[0] - sum(room)])[:-1:2]

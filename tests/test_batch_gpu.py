@@ -93,3 +93,18 @@ def test_batch_mixed_tile_configs(gpu):
         got = canon(v, f)
         ref = alone(j.values, j.level, j.method)
         assert np.array_equal(got[0], ref[0]) and np.array_equal(got[1], ref[1])
+
+
+def test_in_place_with_a_gradient(gpu):
+    """A mesh of a batch takes an in-place change by a tracked tensor, as one of a single call does."""
+    import torch
+
+    from isoext_amd.batch import GridJob, mc_batch
+    v = multi_sphere_field((20, 21, 22), 4, seed=2)
+    t = torch.from_numpy(v).cuda()
+    (va, fa), (vb, fb) = mc_batch([GridJob(t), GridJob(t, 0.05)])
+    shift = torch.zeros(3, device="cuda", requires_grad=True)
+    va.add_(shift)
+    va.sum().backward()
+    assert torch.equal(shift.grad, torch.full((3,), float(va.shape[0]), device="cuda"))
+    assert not vb.requires_grad
