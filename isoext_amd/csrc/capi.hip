@@ -736,6 +736,7 @@ struct ItsPending {
     int dev = -1;
     int64_t *h = nullptr;
     bool ready = false;
+    bool open = false;   // not yet waited for
     ~ItsPending() {
         if (ev) (void) hipEventDestroy(ev);
         if (h) (void) hipHostFree(h);
@@ -744,6 +745,10 @@ struct ItsPending {
         int d = -1;
         hipError_t e = hipGetDevice(&d);
         if (e != hipSuccess) return e;
+        // a set that was begun and given up (no memory for its buffers) may
+        // still be about to write its counts, from whatever stream
+        if (open && (e = hipEventSynchronize(ev)) != hipSuccess) return e;
+        open = false;
         if (!h && (e = hipHostMalloc((void **) &h, 2 * sizeof(int64_t), 0)) != hipSuccess) return e;
         if (ev && dev != d) {
             (void) hipEventDestroy(ev);
@@ -837,7 +842,7 @@ int isoext_its_begin(const isoext_grid *g, float level, void *scratch, int64_t s
     HIP_CHECK(iso::its_dense_count_launch(p, st), "intersection count");
     HIP_CHECK(hipMemcpyAsync(g_its_pending.h, p.totals, 2 * sizeof(int64_t), hipMemcpyDeviceToHost, st), "read counts");
     HIP_CHECK(hipEventRecord(g_its_pending.ev, st), "intersection count");
-    g_its_pending.ready = true;
+    g_its_pending.ready = g_its_pending.open = true;
     return ISOEXT_OK;
 }
 
@@ -858,6 +863,7 @@ int isoext_its_finish(const isoext_grid *g, float level, void *scratch, int64_t 
     o.apre_tab = apre_tab;
     HIP_CHECK(iso::its_dense_emit_launch(iso::mc_auto_config(g->shape), p, o, st), "intersection emit");
     HIP_CHECK(hipEventSynchronize(g_its_pending.ev), "intersection count");
+    g_its_pending.open = false;
     counts[0] = g_its_pending.h[0];
     counts[1] = g_its_pending.h[1];
     if (counts[0] > 0x7fffffffll) return fail(ISOEXT_E_TOO_LARGE, "more than 2^31-1 active cells");

@@ -142,3 +142,33 @@ def test_grids_without_a_cell_in_turn(gpu, monkeypatch):
         a, b = iso.dual_contouring(g, 0.03)
         assert len(runs) == run
         assert a is None and b is None if g is none else torch.equal(a, v) and torch.equal(b, f)
+
+
+def test_begun_and_given_up(gpu, monkeypatch):
+    """A set that was begun and given up has written its counts before the thread's next one is begun, on any stream."""
+    import torch
+
+    import isoext_amd as iso
+    from isoext_amd import dc
+    a, b = (iso.UniformGrid.wrap(torch.from_numpy(field("spheres", s)).cuda()) for s in ((30, 31, 32), (20, 21, 22)))
+    ref = counted(b, 0.0, True)
+    iso.get_intersection(a, 0.0, True)
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    for s in (first, second):   # workspaces, tables
+        with torch.cuda.stream(s):
+            iso.get_intersection(b, 0.0, True)
+    torch.cuda.synchronize()
+
+    def no_memory(*args):
+        raise MemoryError
+
+    with monkeypatch.context() as m, torch.cuda.stream(first):
+        torch.cuda._sleep(5_000_000)
+        m.setattr(dc, "_its_buffers", no_memory)
+        with pytest.raises(MemoryError):
+            iso.get_intersection(a, 0.0, True)
+    with torch.cuda.stream(second):
+        its = iso.get_intersection(b, 0.0, True)
+    assert first.query()
+    torch.cuda.synchronize()
+    assert torch.equal(its.points, ref.points) and torch.equal(its.cell_offsets, ref.cell_offsets)
