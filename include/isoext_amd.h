@@ -342,6 +342,14 @@ int isoext_mc_sparse_run(const isoext_grid *g, float level, int method, const vo
                          const int64_t case_counts[2], void *workspace, int64_t workspace_bytes, float *out_v,
                          int64_t cap_v, int32_t *out_f, int64_t cap_f, int64_t *vsrc, float *vjac,
                          int64_t counts[2], void *stream);
+/* Only the outputs, after isoext_mc_sparse_run came back with
+ * ISOEXT_E_CAPACITY (as it does for out_v and out_f NULL and no room): the
+ * same arguments, scratch and workspace as they are, buffers of exactly the
+ * counts it returned. */
+int isoext_mc_sparse_emit(const isoext_grid *g, float level, int method, const void *scratch,
+                          const int64_t case_counts[2], void *workspace, int64_t workspace_bytes,
+                          const int64_t counts[2], float *out_v, int32_t *out_f, int64_t *vsrc, float *vjac,
+                          void *stream);
 
 /* ---- captured plans (no reference counterpart: repeated extractions of one
  * grid buffer, e.g. an optimisation loop that updates the values in place) ----

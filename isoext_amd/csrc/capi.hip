@@ -1701,6 +1701,24 @@ int isoext_mc_sparse_run(const isoext_grid *g, float level, int method, const vo
     return ISOEXT_OK;
 }
 
+int isoext_mc_sparse_emit(const isoext_grid *g, float level, int method, const void *scratch,
+                          const int64_t case_counts[2], void *workspace, int64_t workspace_bytes,
+                          const int64_t counts[2], float *out_v, int32_t *out_f, int64_t *vsrc, float *vjac,
+                          void *stream) {
+    if (method != 0 && method != 1) return fail(ISOEXT_E_ARG, "Unknown method: %d", method);
+    AABB_CHECK(g->aabb_min, g->aabb_max);
+    const int64_t ninst = case_counts[0], nact = case_counts[1];
+    if (!g->sparse_cell_ids || g->n_sparse == 0 || ninst == 0 || counts[0] == 0) return ISOEXT_OK;
+    if (!out_v || !out_f) return fail(ISOEXT_E_ARG, "output buffer is null");
+    if (workspace_bytes < isoext_mc_sparse_run_bytes(ninst, nact))
+        return fail(ISOEXT_E_WORKSPACE, "sparse marching cubes workspace too small");
+    const iso::SparseMcOut o{out_v, counts[0], out_f, counts[1], vsrc, (float2 *) vjac};
+    HIP_CHECK(iso::sparse_mc_emit(smc_in(g, level, method), scratch, ninst, nact, workspace, (size_t) workspace_bytes,
+                                  o, (hipStream_t) stream),
+              "sparse marching cubes");
+    return ISOEXT_OK;
+}
+
 int isoext_mc_sparse_count(const isoext_grid *g, float level, int64_t *scratch, int64_t *ninst, void *stream) {
     *ninst = 0;
     AABB_CHECK(g->aabb_min, g->aabb_max);

@@ -77,7 +77,11 @@ size_t sparse_mc_run_bytes(int64_t ninst, int64_t nact);
 hipError_t sparse_mc_cases(const SparseMcIn &in, void *scratch, int64_t &ninst, int64_t &nact, hipStream_t st);
 hipError_t sparse_mc_run(const SparseMcIn &in, const void *scratch, int64_t ninst, int64_t nact, void *work,
                          size_t work_bytes, SparseMcOut &o, int64_t &nv, int64_t &nf, hipStream_t st);
-// The same with nothing kept between the count and the run (the cases are
+// Vertices and faces of a run that found too little room for them (nothing in
+// between): o has room for the sizes it returned.
+hipError_t sparse_mc_emit(const SparseMcIn &in, const void *scratch, int64_t ninst, int64_t nact, void *work,
+                          size_t work_bytes, const SparseMcOut &o, hipStream_t st);
+// Both steps with nothing kept between the count and the run (the cases are
 // found twice): scratch of the count 8 * (n / 256 + 16) bytes.
 size_t sparse_mc_work_bytes(int64_t n, int64_t ninst);
 hipError_t sparse_mc_count(const SparseMcIn &in, int64_t *scratch, int64_t &ninst, hipStream_t st);

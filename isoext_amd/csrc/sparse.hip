@@ -1186,26 +1186,39 @@ hipError_t read2(const int64_t *src, int64_t out[2], hipStream_t st) {
     return hipSuccess;
 }
 
-size_t mc_work_bytes(int64_t ninst, int64_t na) {
-    const int64_t nblk = nb(na), nch = (nblk + kScanBlk - 1) / kScanBlk;
-    size_t b = 0;
-    auto add = [&](size_t x) { b += (x + 255) & ~size_t(255); };
-    add(8 * na);              // aid
-    add(4 * na);              // aslot
-    add(8 * na);              // ainfo
-    add(4 * na);              // ares
-    add(4 * na);              // alook
-    add(12 * nblk);           // win
-    add(8 * nblk);            // bid
-    add(4 * ninst);           // rkey
-    add(4 * ninst);           // vid
-    add(ninst + 16);          // used
-    add(8 * nblk);            // block sums
-    add(16 * nch);            // chunk sums
-    add(16 * nblk);           // block prefixes
-    add(16);                  // totals
-    return b;
-}
+// Workspace of a run.
+struct RunWork {
+    SparseMcWork w;
+    uint2 *bsum;             // per workgroup: vertices, faces
+    longlong2 *chunk, *pre;  // their chunk sums and prefixes
+    int64_t *tot;
+    size_t bytes;
+    RunWork(void *base, int64_t ninst, int64_t na) {
+        const size_t nblk = nb(na), nch = (nblk + kScanBlk - 1) / kScanBlk;
+        bytes = 0;
+        auto take = [&](size_t n) {
+            char *r = (char *) base + bytes;
+            bytes += (n + 255) & ~size_t(255);
+            return r;
+        };
+        w.aid = (int64_t *) take(8 * na);
+        w.aslot = (int32_t *) take(4 * na);
+        w.ainfo = (uint2 *) take(8 * na);
+        w.ares = (uint32_t *) take(4 * na);
+        w.alook = (uint32_t *) take(4 * na);
+        w.win = (int32_t *) take(12 * nblk);
+        w.bid = (int64_t *) take(8 * nblk);
+        w.rkey = (int32_t *) take(4 * ninst);
+        w.vid = (int32_t *) take(4 * ninst);
+        w.used = (uint8_t *) take(ninst + 16);
+        bsum = (uint2 *) take(8 * nblk);
+        chunk = (longlong2 *) take(16 * nch);
+        pre = (longlong2 *) take(16 * nblk);
+        tot = (int64_t *) take(16);
+    }
+};
+
+size_t mc_work_bytes(int64_t ninst, int64_t na) { return RunWork(nullptr, ninst, na).bytes; }
 
 }   // namespace
 
@@ -1250,28 +1263,8 @@ hipError_t sparse_mc_run(const SparseMcIn &in, const void *scratch, int64_t nins
     ISO_TRY(sparse_mc_luts());
     const CaseScratch c(const_cast<void *>(scratch), in.n, true);
     const unsigned nblk = nb(nact);
-    const int64_t nch = ((int64_t) nblk + kScanBlk - 1) / kScanBlk;
-    char *p = (char *) work;
-    auto take = [&](size_t n) {
-        char *r = p;
-        p += (n + 255) & ~size_t(255);
-        return r;
-    };
-    SparseMcWork w;
-    w.aid = (int64_t *) take(8 * nact);
-    w.aslot = (int32_t *) take(4 * nact);
-    w.ainfo = (uint2 *) take(8 * nact);
-    w.ares = (uint32_t *) take(4 * nact);
-    w.alook = (uint32_t *) take(4 * nact);
-    w.win = (int32_t *) take(12 * (size_t) nblk);
-    w.bid = (int64_t *) take(8 * (size_t) nblk);
-    w.rkey = (int32_t *) take(4 * ninst);
-    w.vid = (int32_t *) take(4 * ninst);
-    w.used = (uint8_t *) take(ninst + 16);
-    uint2 *bsum = (uint2 *) take(8 * (size_t) nblk);
-    longlong2 *chunk = (longlong2 *) take(16 * nch);
-    longlong2 *pre = (longlong2 *) take(16 * (size_t) nblk);
-    int64_t *tot = (int64_t *) take(16);
+    const RunWork r(work, ninst, nact);
+    const SparseMcWork &w = r.w;
 
     const int64_t ncell = (in.n + kCellBlk - 1) / kCellBlk, nu = (ninst + 15) / 8;
     hipLaunchKernelGGL(k_fill_u64, dim3(gs(nu)), dim3(kB), 0, st, (unsigned long long *) w.used, nu, 0ull);
@@ -1282,18 +1275,28 @@ hipError_t sparse_mc_run(const SparseMcIn &in, const void *scratch, int64_t nins
     hipLaunchKernelGGL(k_smc_special, dim3((unsigned) ((nact + kSpecBlk - 1) / kSpecBlk)), dim3(kB), 0, st, in, w,
                        (const int64_t *) c.tot);
     hipLaunchKernelGGL(k_smc_sizes, dim3((nblk + kB / 64 - 1) / (kB / 64)), dim3(kB), 0, st, w, (const int64_t *) c.tot,
-                       (int64_t) nblk, bsum);
-    scan_pairs(bsum, nblk, chunk, pre, tot, st);
+                       (int64_t) nblk, r.bsum);
+    scan_pairs(r.bsum, nblk, r.chunk, r.pre, r.tot, st);
     ISO_TRY(hipGetLastError());
     int64_t h[2];
-    ISO_TRY(read2(tot, h, st));
+    ISO_TRY(read2(r.tot, h, st));
     nv = h[0];
     nf = h[1];
-    if (nv > o.cap_v || nf > o.cap_f) return hipSuccess;   // caller re-allocates and retries
-    hipLaunchKernelGGL(k_smc_verts, dim3(nblk), dim3(kB), 0, st, in, w, (const int64_t *) c.tot,
-                       (const longlong2 *) pre, o);
-    hipLaunchKernelGGL(k_smc_faces, dim3((nblk + 7) / 8 * 8), dim3(kB), 0, st, in, w, (const int64_t *) c.tot,
-                       (const longlong2 *) pre, o);
+    if (nv > o.cap_v || nf > o.cap_f) return hipSuccess;   // caller makes room: sparse_mc_emit, or the run again
+    return sparse_mc_emit(in, scratch, ninst, nact, work, work_bytes, o, st);
+}
+
+hipError_t sparse_mc_emit(const SparseMcIn &in, const void *scratch, int64_t ninst, int64_t nact, void *work,
+                          size_t work_bytes, const SparseMcOut &o, hipStream_t st) {
+    if (in.n == 0 || ninst == 0) return hipSuccess;
+    if (mc_work_bytes(ninst, nact) > work_bytes) return hipErrorInvalidValue;
+    const CaseScratch c(const_cast<void *>(scratch), in.n, true);
+    const RunWork r(work, ninst, nact);
+    const unsigned nblk = nb(nact);
+    hipLaunchKernelGGL(k_smc_verts, dim3(nblk), dim3(kB), 0, st, in, r.w, (const int64_t *) c.tot,
+                       (const longlong2 *) r.pre, o);
+    hipLaunchKernelGGL(k_smc_faces, dim3((nblk + 7) / 8 * 8), dim3(kB), 0, st, in, r.w, (const int64_t *) c.tot,
+                       (const longlong2 *) r.pre, o);
     ISO_TRY(hipGetLastError());
     ISO_TRY(hipStreamSynchronize(st));
     return hipSuccess;

@@ -37,6 +37,8 @@ _lib.declare("isoext_mc_sparse_run_bytes", i64, [i64, i64])
 _lib.declare("isoext_mc_sparse_cases", ctypes.c_int, [vp, f32, vp, i64, i64 * 2, vp])
 _lib.declare("isoext_mc_sparse_run", ctypes.c_int, [vp, f32, ctypes.c_int, vp, i64 * 2, vp, i64, vp, i64, vp, i64, vp,
                                                     vp, i64 * 2, vp])
+_lib.declare("isoext_mc_sparse_emit", ctypes.c_int, [vp, f32, ctypes.c_int, vp, i64 * 2, vp, i64, i64 * 2, vp, vp, vp,
+                                                     vp, vp])
 _lib.declare("isoext_sparse_setop_scratch_bytes", i64, [i64, i64])
 _lib.declare("isoext_sparse_union", ctypes.c_int, [vp, i64, vp, i64, vp, i64, vp, vp, vp, vp])
 _lib.declare("isoext_sparse_difference", ctypes.c_int, [vp, i64, vp, i64, vp, i64, vp, vp, vp, vp])
@@ -222,6 +224,12 @@ def grid_struct_of(grid):
     return grid_struct(grid)
 
 
+# Crossing edges of the cells (about four a vertex) from which outputs that are
+# kept for a backward pass get buffers of their own size, made between the count
+# and the output (15 us); below, buffers for all of them hold 10 MB at most.
+_EXACT_FROM = 1 << 18
+
+
 def mc_sparse(grid: SparseGrid, level: float, method: int, want_src: bool = False, want_jac: bool = False):
     """Marching cubes over a sparse grid; returns (v, f[, vsrc[, vjac]]):
     vsrc the slot * 12 + edge of each vertex, vjac ((V, 2) float32) the
@@ -244,17 +252,25 @@ def mc_sparse(grid: SparseGrid, level: float, method: int, want_src: bool = Fals
         if ni == 0:
             return empty
         ws = workspace.get("sparse_mc", L.isoext_mc_sparse_run_bytes(ni, na), dev)
-        cap_v, cap_f = ni, 5 * na
         counts = (ctypes.c_int64 * 2)()
+        args = (ctypes.byref(g), float(level), int(method), scratch.data_ptr(), case_counts, ws.data_ptr(), ws.numel())
+        cap_v, cap_f = ni, 5 * na
+        exact = want_jac and ni > _EXACT_FROM
+        if exact:
+            rc = L.isoext_mc_sparse_run(*args, None, 0, None, 0, None, None, counts, stream)
+            if rc != _lib.E_CAPACITY:
+                _lib.check(rc, "marching_cubes")
+            cap_v, cap_f = int(counts[0]), int(counts[1])
         for _ in range(2):
             v = torch.empty((max(cap_v, 1), 3), dtype=torch.float32, device=dev)
             f = torch.empty((max(cap_f, 1), 3), dtype=torch.int32, device=dev)
             src = torch.empty(max(cap_v, 1), dtype=torch.int64, device=dev) if want_src or want_jac else None
             jac = torch.empty((max(cap_v, 1), 2), dtype=torch.float32, device=dev) if want_jac else None
-            rc = L.isoext_mc_sparse_run(ctypes.byref(g), float(level), int(method), scratch.data_ptr(), case_counts,
-                                        ws.data_ptr(), ws.numel(), v.data_ptr(), cap_v, f.data_ptr(), cap_f,
-                                        src.data_ptr() if src is not None else None,
-                                        jac.data_ptr() if jac is not None else None, counts, stream)
+            ps, pj = (t.data_ptr() if t is not None else None for t in (src, jac))
+            if exact:
+                rc = L.isoext_mc_sparse_emit(*args, counts, v.data_ptr(), f.data_ptr(), ps, pj, stream)
+            else:
+                rc = L.isoext_mc_sparse_run(*args, v.data_ptr(), cap_v, f.data_ptr(), cap_f, ps, pj, counts, stream)
             if rc == _lib.E_CAPACITY:
                 cap_v, cap_f = int(counts[0]), int(counts[1])
                 continue

@@ -113,3 +113,24 @@ def test_one_step_abi_and_gradients(gpu, shape, keep, kind):
         term.index_add_(0, 8 * (src // 12) + corner[k][e], ga * jac[:, k].double().nan_to_num(0.0, 0.0, 0.0).abs())
     bound = 16 * 2.0 ** -24 * term.view_as(a) + 1e-37
     assert bool(((a.double() - b.double()).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("n", [16, 44])   # below and above the crossing edges from which buffers are made to size
+def test_what_is_kept_for_backward(gpu, n):
+    """Large results are kept at their own size, and are those of a call with room for every crossing edge."""
+    import torch
+
+    from isoext_amd import autograd
+    from isoext_amd.sparse import mc_sparse
+    shape, rng = (n, n + 1, n + 2), np.random.default_rng(n)
+    ids = cells_of(shape, 1.0, rng)
+    grid = make(shape, ids, corner_values(rng.standard_normal(shape), ids))
+    values = grid.values.clone().requires_grad_()
+    v, f = autograd.marching_cubes(grid, values, 0.0)
+    src, jac = v.grad_fn.saved_tensors[1:]
+    v2, f2, src2 = mc_sparse(grid, 0.0, 0, want_src=True)
+    assert torch.equal(v.detach(), v2) and torch.equal(f, f2) and torch.equal(src, src2)
+    kept = sum(t.untyped_storage().nbytes() for t in (src, jac))
+    assert kept <= (16 * v.shape[0] if n == 44 else 16 << 18)
+    (g,) = torch.autograd.grad(v.sum(), values)
+    assert bool(g.isfinite().all()) and g.abs().sum() > 0
