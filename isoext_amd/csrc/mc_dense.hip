@@ -2416,20 +2416,30 @@ int64_t mc_config_tiles(int cfg, const int64_t shape[3]) {
 
 // First tile in the order that still gives every CU several workgroups
 // (16x16x64 cells from about 384^3 up, 8x8x64 near 256^3); when none does,
-// the one with the most tiles (4x4x64).  On a small grid the emit is one
-// round of workgroups and takes as long as its fullest tile: quarter tiles
-// halve the cells that one workgroup walks one batch after another (whole
-// call 8x8x64 -> 4x4x64: 64^3 49.0 -> 45.5 us, 128^3 62.3 -> 55.3, 192^3
-// with 1728 8x8x64 tiles 60.9 -> 58.5), while from 2048 tiles on the halo
-// read again by each tile costs more (224^3, 3136 tiles, 79.8 -> 88.3;
-// 256^3 125 -> 141).  128 threads a tile: 64^3 45.1, 160^3 61.9 instead of
-// 60.0; 64 threads 51.5 at 64^3.  With empty tiles skipped through the
+// the one with the most tiles.  With empty tiles skipped through the
 // active-tile list, 16x16x64 extracted fastest at 384^3..1024^3 on MI355X
 // (0.5-8% ahead of 16x16x128, which never has more tiles and so is not in
 // the order); 16x16x256 never wins.
+//
+// 4x4x64 on small grids: their emit is one round of workgroups and takes as
+// long as its fullest tile, and quarter tiles halve the cells that one
+// workgroup walks one batch after another.  That holds up to two 8x8x64 tiles
+// a CU, and where such a tile has more cells than a batch (256).  Whole calls,
+// 8x8x64 -> 4x4x64, 64 spheres: 100^3 70.8 -> 62.5 us, 128^3 (512 tiles)
+// 74.3 -> 67.8, 160x160x33 62.4 -> 60.2; beyond, the halo that each tile reads
+// again costs more: 200x200x33 (625 tiles) 66.6 -> 71.1, 256x256x65 72.7 ->
+// 82.5, 192^3 84.3 -> 92.9.  Thin tiles, noise: 120x120x6 (320 cells) 73.2 ->
+// 69.9, 120x120x5 (256) 55.3 -> 56.7, 300x300x2 76.6 -> 106.9.  The tiles of
+// an intersection pass alone (8 spheres): 64^3 25.6 -> 19.4, 128^3 28.6 ->
+// 21.4 us.  128 threads a tile: 64^3 45.1 instead of 45.5 us, 160^3 61.9
+// instead of 60.0; 64 threads 51.5 at 64^3.
 int mc_auto_config(const int64_t shape[3]) {
-    static const int order[] = {3, 1, 5, 7};
-    constexpr int64_t kWant = 2048;
+    static const int order[] = {3, 1, 5};
+    constexpr int64_t kWant = 2048, kSmall = 512, kBatchCells = 256;
+    const int64_t tiles8 = mc_config_tiles(5, shape);
+    const int64_t cells8 = std::min<int64_t>(shape[0] - 1, 8) * std::min<int64_t>(shape[1] - 1, 8) *
+                           std::min<int64_t>(shape[2] - 1, 64);
+    if (tiles8 > 0 && tiles8 <= kSmall && cells8 > kBatchCells) return 7;
     int best = 0;
     int64_t best_tiles = -1;
     for (int cfg : order) {

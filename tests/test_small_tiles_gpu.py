@@ -11,13 +11,20 @@ from test_mc_dense_gpu import assert_same_mesh, run_gpu
 SMALL, WIDE = 7, 5
 
 
-def test_rule():
-    from isoext_amd import _lib
-    auto = _lib.lib().isoext_mc_auto_config
-    assert auto(_lib.i64x3((18, 5, 2))) == auto(_lib.i64x3((192, 192, 192))) == SMALL
-    # 27 * 26 * 3 = 2106 tiles of 8 x 8 x 64, 26 * 26 * 3 = 2028
-    assert auto(_lib.i64x3((217, 209, 193))) == WIDE
-    assert auto(_lib.i64x3((209, 209, 193))) == SMALL
+# at most 512 tiles of 8 x 8 x 64 cells, of more than 256 cells each: (18, 5, 2) has tiles of 8 x 4 x 1,
+# 128^3 512 tiles, (129, 137, 129) 544, (120, 120, 5) tiles of 256 cells and (120, 120, 6) of 320; flat grids and
+# larger ones keep the wide tiles
+@pytest.mark.parametrize("shape,small", [
+    ((64, 64, 64), True), ((97, 131, 75), True), ((128, 128, 128), True), ((129, 129, 129), True),
+    ((129, 137, 129), False), ((120, 120, 6), True), ((120, 120, 5), False), ((160, 160, 33), True),
+    ((200, 200, 33), False), ((362, 362, 2), False), ((300, 400, 2), False), ((2, 8192, 16), False),
+    ((2, 1024, 128), True), ((2, 2049, 129), True), ((2, 2058, 129), False), ((192, 192, 192), False),
+    ((256, 256, 65), False), ((18, 5, 2), False), ((2, 2, 2), False), ((10, 10, 10), True)])
+def test_rule(shape, small):
+    """What marching cubes takes (table or rule) and what intersections take (the rule)."""
+    from isoext_amd import _lib, autotune
+    assert (_lib.lib().isoext_mc_auto_config(_lib.i64x3(shape)) == SMALL) == small
+    assert (autotune.mc_config(shape) == SMALL) == small
 
 
 # noise fills tiles (1024 cells, four rounds of a workgroup), ties weld
