@@ -229,7 +229,7 @@ def _remember(hints, shape, sizes, low=None):
     fall by a 32nd a call.  With the eighth more that the next call makes room
     for, a large surface still fits after three small ones of its shape (too
     little room costs a second run), and a lone large one is soon forgotten.
-    low: the same of the last size from the other side."""
+    low: the last size from the other side, an eighth of the way a call."""
     with _hint_lock:
         if len(hints) > 4096:
             hints.clear()
@@ -238,7 +238,7 @@ def _remember(hints, shape, sizes, low=None):
             if len(low) > 4096:
                 low.clear()
             o = low.get(shape, sizes[-1])
-            low[shape] = min(sizes[-1], o + o // 32 + 32)
+            low[shape] = min(sizes[-1], o + (sizes[-1] - o + 7) // 8)
 
 
 def _its_vary(shape):

@@ -49,3 +49,18 @@ def test_grid_workspace_per_cell():
     size = _lib.lib().isoext_dc_grid_workspace_bytes
     n = 1 << 20
     assert (size(ctypes.byref(g), 2 * n) - size(ctypes.byref(g), n)) / n < 60
+
+
+def test_sizes_that_vary(monkeypatch):
+    """Counted first only while small sets are among the recent ones: a steady size is guessed again soon, also after
+    empty sets."""
+    for name in ("_its_hint", "_its_low"):
+        monkeypatch.setattr(dc, name, {})
+    shape, vary = (200, 200, 200), []
+    for n in [0, 0] + [400_000] * 9 + [2_000] + [400_000] * 9:
+        vary.append(dc._its_vary(shape))
+        dc._remember(dc._its_hint, shape, (n // 4, n), dc._its_low)
+    assert not any(vary[:3]) and all(vary[3:5]) and not any(vary[9:12]) and all(vary[12:14]) and not any(vary[18:])
+    for _ in range(200):   # a lone large set is forgotten
+        dc._remember(dc._its_hint, shape, (500, 2_000), dc._its_low)
+    assert not dc._its_vary(shape) and dc._its_caps(shape)[1] < 20_000
