@@ -40,6 +40,7 @@ struct SparseMcWork {
     uint2 *ainfo;      // its first instance; case, special flag, crossing edges
     uint32_t *ares;    // edges that represent themselves, kept faces, special flag
     uint32_t *alook;   // edges whose vertex may lie near a grid point
+    int4 *acol;        // of those with such an edge: places in the list of columns (-1, -1), (-1, 0), (-1, 1), (0, -1)
     int32_t *win;      // per workgroup: the runs of active cells its cells' lower neighbours are in
     int64_t *bid;      // first id of each workgroup's active cells
     int32_t *rkey;     // per instance: its representative (first instance at its position)

@@ -449,34 +449,68 @@ __device__ __forceinline__ int near_end(const SparseMcIn &in, const SparseMcWork
 }
 
 // By position, the first (active cell, edge) that holds the vertex of edge e
-// of active cell a, a vertex within 16 ulps of corner pc of the cell: among
-// the edges through that grid point in the cell that lane d of eight looks
-// at.  Searches the runs of the cell's workgroup.  Returns the active cell *
-// 16 + edge.
-__device__ __forceinline__ int64_t rep_at_point(const SparseMcIn &in, const SparseMcWork &w, int64_t a, int e, int d,
+// of active cell a, a vertex within 16 ulps of corner pc of the cell: the edges
+// through that grid point in the cells around it, in id order up to this one.
+// Each is in one of the four columns whose places in the active list
+// k_smc_link left (w.acol), a step or two from there.  Returns the active
+// cell * 16 + edge.
+__device__ __forceinline__ int64_t rep_at_point(const SparseMcIn &in, const SparseMcWork &w, int64_t a, int e,
                                                 int pc) {
-    const int64_t cy = in.g.Y - 1, cz = in.g.Z - 1, id = w.aid[a], s = w.aslot[a];
-    const int32_t *win = w.win + 3 * (a / kB);
-    int64_t x, y, z;
-    cell_xyz(in, id, x, y, z);
-    float px = 0.f, py = 0.f, pz = 0.f;
-    inst_pos(in, s, x, y, z, e, px, py, pz);
-    int64_t best = a * 16 + e;
-    const int64_t xx = x + (pc >> 2) - (d >> 2), yy = y + ((pc >> 1) & 1) - ((d >> 1) & 1), zz = z + (pc & 1) - (d & 1);
-    if (xx < 0 || yy < 0 || zz < 0 || yy >= cy || zz >= cz) return best;
-    const int64_t key = (xx * cy + yy) * cz + zz;
-    if (key > id) return best;   // only the cells up to this one
-    const bool before = xx < x;
-    const int64_t hi = before ? win[1] : a + 1, p = lower_id(w.aid, before ? win[0] : win[2], hi, key);
-    if (p >= hi || w.aid[p] != key) return best;
-    const int64_t sp = w.aslot[p];
-    for (int a2 = 0; a2 < 3; ++a2) {
-        const int e2 = edge_of(d & ~(4 >> a2), a2);
-        if (p * 16 + e2 >= best) continue;
-        float qx, qy, qz;
-        if (inst_pos(in, sp, xx, yy, zz, e2, qx, qy, qz) && qx == px && qy == py && qz == pz) best = p * 16 + e2;
+    const int64_t cy = in.g.Y - 1, cz = in.g.Z - 1, id = w.aid[a];
+    const int4 col = w.acol[a];
+    int64_t o[3];
+    cell_xyz(in, id, o[0], o[1], o[2]);
+    const int64_t n[3] = {in.g.X, in.g.Y, in.g.Z};
+    float g[3][3];   // coordinates around the point, by axis
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+        const int64_t q = o[u] + ((pc >> (2 - u)) & 1);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) g[u][k] = grid_coord(q + k - 1, n[u], in.g.amin[u], in.g.amax[u]);
     }
-    return best;
+    // position of the vertex on the edge along axis ax that ends (hi) or begins at the point
+    auto place = [&](const float *v, int c, int ax, float p[3]) {
+        const int bit = 4 >> ax;
+        const bool hi = c & bit;   // c: the point as a corner of the cell with values v
+        const float va = v[c & ~bit], vb = v[c | bit];
+        if (inside(va, in.level) == inside(vb, in.level)) return false;
+        const float t = edge_t(va, vb, in.level);
+#pragma unroll
+        for (int u = 0; u < 3; ++u)
+            p[u] = u == ax ? lerp1(t, hi ? g[u][0] : g[u][1], hi ? g[u][1] : g[u][2]) : lerp1(t, g[u][1], g[u][1]);
+        return true;
+    };
+    float pos[3] = {0.f, 0.f, 0.f};
+    place(in.values + 8 * (int64_t) w.aslot[a], pc, edge_axis(e), pos);
+    for (int d = 7; d >= 0; --d) {   // the point is corner d of the cell looked at
+        const int dx = (pc >> 2) - (d >> 2), dy = ((pc >> 1) & 1) - ((d >> 1) & 1), dz = (pc & 1) - (d & 1);
+        const int64_t xx = o[0] + dx, yy = o[1] + dy, zz = o[2] + dz;
+        if (xx < 0 || yy < 0 || zz < 0 || yy >= cy || zz >= cz) continue;
+        const int64_t key = (xx * cy + yy) * cz + zz;
+        if (key > id) break;
+        // columns (-1, -1) and (-1, 1) from this cell's z on, (-1, 0) and (0, -1) from z - 1 on, its own: itself or
+        // the one before it
+        int64_t p = a;
+        int steps = dz;
+        if (dx < 0 || dy < 0) {
+            const bool from_z = dx < 0 && dy != 0;
+            p = from_z ? (dy < 0 ? col.x : col.z) : (dx < 0 ? col.y : col.w);
+            if (!from_z) ++steps;
+        }
+        if (steps < 0) --p;
+        for (; steps > 0 && p < a && w.aid[p] < key; --steps) ++p;
+        if (p < 0 || p > a || (p == a ? id : w.aid[p]) != key) continue;
+        const float *v = in.values + 8 * (int64_t) w.aslot[p];
+        int first = 16;
+#pragma unroll
+        for (int ax = 0; ax < 3; ++ax) {
+            float q[3];
+            const int e2 = edge_of(d & ~(4 >> ax), ax);
+            if (place(v, d, ax, q) && q[0] == pos[0] && q[1] == pos[1] && q[2] == pos[2]) first = min(first, e2);
+        }
+        if (first < (p == a ? e : 16)) return p * 16 + first;
+    }
+    return a * 16 + e;
 }
 
 // One workgroup per kB active cells.  The lower neighbours of its cells lie
@@ -702,28 +736,39 @@ __global__ void __launch_bounds__(kB) k_smc_link(SparseMcIn in, SparseMcWork w, 
     const uint64_t tw = cSTris[in.method][info.y & 255];
     w.ares[a] = own | ((1u << (tw & 15)) - 1) << 12 | (info.y & kSpecial ? kResSpecial : 0u);
     w.alook[a] = look;
+    if (look) w.acol[a] = make_int4((int) nbi[0], (int) nbi[1], (int) nbi[4], (int) nbi[5]);
 }
 
-// The edges whose vertex may lie near a grid point: a workgroup takes
-// kSpecBlk active cells, lists those edges in LDS, one lane tests each, and
-// eight lanes find the representative of one that is near by position.  Then
-// the cells that had any: faces with two corners at one position are dropped,
-// the kept ones mark the vertices they use.  A chain of dependent loads for
-// few edges: many cells a workgroup, so that each step of the chain serves
-// many of them at once (kSpecBlk 512: 226 us, 1024: 147 us at 9.7 M active
-// cells, most of it the chain).
+// The edges whose vertex may lie near a grid point: a workgroup takes `per`
+// active cells, lists those edges in LDS, one lane tests each, and one lane
+// finds the representative of one that is near by position.  Then the cells
+// that had any: faces with two corners at one position are dropped, the kept
+// ones mark the vertices they use.
+//
+// With few such edges it is a chain of dependent loads: many cells a
+// workgroup, so that each step of the chain serves many of them at once (per =
+// 512: 226 us, 1024: 147, 4096: 138 at 9.7 M active cells, most of it the
+// chain).  Where many corners are at the level, it is the work at those edges,
+// and it has to fill the chip: 2048 workgroups before any takes more than kB
+// cells.  One lane an edge, from the lowest cell around the point to the first
+// that matches, with the columns' places from k_smc_link and nine coordinates
+// worked out once: eight lanes with a search and all their own coordinates
+// each took six times as long.  Fields rounded to a cell: 200^3 (19 k active
+// cells, 4096 a workgroup) 2.06 -> 0.05 ms, the 2048^3 band (9.7 M active
+// cells, a quarter of the corners at the level) 10.3 -> 1.85 ms.
+constexpr int64_t kSpecWgs = 2048;
 constexpr int kSpecBlk = 4096, kSpecCells = 1024, kSpecList = 2048;
-__global__ void __launch_bounds__(kB) k_smc_special(SparseMcIn in, SparseMcWork w, const int64_t *tot) {
+__global__ void __launch_bounds__(kB) k_smc_special(SparseMcIn in, SparseMcWork w, const int64_t *tot, int per) {
     // room for one more round of kB cells above the marks at which the lists are worked off
     __shared__ uint32_t list[kSpecList + 12 * kB];   // cell's place in cells (bits 0-11), edge (12-15), corner (16-18)
     __shared__ uint16_t cells[kSpecCells + kB];
     __shared__ uint32_t own[kSpecCells + kB];
     __shared__ int nlist, ncells, nslow;
-    const int64_t na = tot[0], a0 = (int64_t) blockIdx.x * kSpecBlk;
+    const int64_t na = tot[0], a0 = (int64_t) blockIdx.x * per;
     if (a0 >= na) return;
     if (threadIdx.x == 0) nlist = ncells = nslow = 0;
     __syncthreads();
-    const int nblk = (int) min<int64_t>(kSpecBlk, na - a0);
+    const int nblk = (int) min<int64_t>(per, na - a0);
     for (int c0 = 0; c0 < nblk; c0 += kB) {
         const int c = c0 + threadIdx.x;
         const uint32_t look = c < nblk ? w.alook[a0 + c] : 0u;
@@ -755,22 +800,16 @@ __global__ void __launch_bounds__(kB) k_smc_special(SparseMcIn in, SparseMcWork 
             if (end) list[atomicAdd(&nslow, 1)] = ent;   // at most as many as were read
         }
         __syncthreads();
-        // ... and eight lanes look around each
-        for (int i = threadIdx.x >> 3; i < nslow; i += kB / 8) {
+        // ... and one lane looks around each
+        for (int i = threadIdx.x; i < nslow; i += kB) {
             const int ci = list[i] & 4095, e = (list[i] >> 12) & 15;
-            const int64_t a = a0 + cells[ci];
-            int64_t best = rep_at_point(in, w, a, e, threadIdx.x & 7, list[i] >> 16);
-#pragma unroll
-            for (int o = 4; o >= 1; o >>= 1) best = min(best, (int64_t) __shfl_xor(best, o, 8));
-            if ((threadIdx.x & 7) == 0) {
-                const int64_t ra = best >> 4;
-                const int re = (int) best & 15;
-                const uint2 f = w.ainfo[a], fr = w.ainfo[ra];
-                w.rkey[f.x + edge_rank((int) (f.y >> 16) & 0xfff, e)] =
-                    (int32_t) fr.x + edge_rank((int) (fr.y >> 16) & 0xfff, re);
-                if (ra == a && re == e) atomicOr(&own[ci], 1u << e);
-                else atomicAnd(&own[ci], ~(1u << e));
-            }
+            const int64_t a = a0 + cells[ci], best = rep_at_point(in, w, a, e, list[i] >> 16), ra = best >> 4;
+            const int re = (int) best & 15;
+            const uint2 f = w.ainfo[a], fr = w.ainfo[ra];
+            w.rkey[f.x + edge_rank((int) (f.y >> 16) & 0xfff, e)] =
+                (int32_t) fr.x + edge_rank((int) (fr.y >> 16) & 0xfff, re);
+            if (ra == a && re == e) atomicOr(&own[ci], 1u << e);
+            else atomicAnd(&own[ci], ~(1u << e));
         }
         __threadfence_block();
         __syncthreads();
@@ -1206,6 +1245,7 @@ struct RunWork {
         w.ainfo = (uint2 *) take(8 * na);
         w.ares = (uint32_t *) take(4 * na);
         w.alook = (uint32_t *) take(4 * na);
+        w.acol = (int4 *) take(16 * na);
         w.win = (int32_t *) take(12 * nblk);
         w.bid = (int64_t *) take(8 * nblk);
         w.rkey = (int32_t *) take(4 * ninst);
@@ -1272,8 +1312,9 @@ hipError_t sparse_mc_run(const SparseMcIn &in, const void *scratch, int64_t nins
                        (const longlong2 *) c.pre, w);
     hipLaunchKernelGGL(k_smc_windows, dim3((nblk + 63) / 64), dim3(64), 0, st, in, w, (const int64_t *) c.tot);
     hipLaunchKernelGGL(k_smc_link, dim3((nblk + 7) / 8 * 8), dim3(kB), 0, st, in, w, (const int64_t *) c.tot);
-    hipLaunchKernelGGL(k_smc_special, dim3((unsigned) ((nact + kSpecBlk - 1) / kSpecBlk)), dim3(kB), 0, st, in, w,
-                       (const int64_t *) c.tot);
+    const int per = (int) std::min<int64_t>(kSpecBlk, kB * (nact / (kSpecWgs * kB) + 1));
+    hipLaunchKernelGGL(k_smc_special, dim3((unsigned) ((nact + per - 1) / per)), dim3(kB), 0, st, in, w,
+                       (const int64_t *) c.tot, per);
     hipLaunchKernelGGL(k_smc_sizes, dim3((nblk + kB / 64 - 1) / (kB / 64)), dim3(kB), 0, st, w, (const int64_t *) c.tot,
                        (int64_t) nblk, r.bsum);
     scan_pairs(r.bsum, nblk, r.chunk, r.pre, r.tot, st);

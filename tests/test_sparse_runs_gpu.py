@@ -115,13 +115,32 @@ def test_one_step_abi_and_gradients(gpu, shape, keep, kind):
     assert bool(((a.double() - b.double()).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("shape,kind", [((92, 86, 80), "ties"), ((90, 2, 3400), "ties"), ((3, 420, 500), "lone")])
+def test_many_vertices_at_grid_points(gpu, shape, kind):
+    """Enough active cells for workgroups of more than 256 of them, with vertices at grid points in most cells, or in a
+    few at the ends of columns and slabs: the first cell of every position by the oracle."""
+    import isoext_amd as iso
+    rng = np.random.default_rng(shape)
+    ids = cells_of(shape, 0.98, rng)
+    field = np.round(rng.standard_normal(shape) * 1.5)
+    if kind == "lone":
+        field = np.where(field == 0, 0.37, field)
+        field[0, 0, 0] = field[1, -1, -1] = field[2, 0, -1] = field[1, 7, 0] = field[-1, -1, 5] = 0.0
+    vals = corner_values(field, ids)
+    v, f = iso.marching_cubes(make(shape, ids, vals), 0.0)
+    a, b = oracle.canonical(*oracle.mc_sparse(ids, vals, shape, 0.0, "nagae")), oracle.canonical(v.cpu().numpy(),
+                                                                                                  f.cpu().numpy())
+    assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+
+
 @pytest.mark.parametrize("n", [16, 44])   # below and above the crossing edges from which buffers are made to size
-def test_what_is_kept_for_backward(gpu, n):
+def test_what_is_kept_for_backward(gpu, monkeypatch, n):
     """Large results are kept at their own size, and are those of a call with room for every crossing edge."""
     import torch
 
-    from isoext_amd import autograd
+    from isoext_amd import autograd, sparse
     from isoext_amd.sparse import mc_sparse
+    monkeypatch.setattr(sparse, "_EXACT_FROM", 1 << 18, raising=False)
     shape, rng = (n, n + 1, n + 2), np.random.default_rng(n)
     ids = cells_of(shape, 1.0, rng)
     grid = make(shape, ids, corner_values(rng.standard_normal(shape), ids))
