@@ -226,8 +226,9 @@ def grid_struct_of(grid):
 
 # Crossing edges of the cells (about four a vertex) from which outputs that are
 # kept for a backward pass get buffers of their own size, made between the count
-# and the output (15 us); below, buffers for all of them hold 10 MB at most.
-_EXACT_FROM = 1 << 18
+# and the output (20 us of 1700 at 39 M edges); below, what is kept takes 64 MB at
+# most.
+_EXACT_FROM = 1 << 22
 
 
 def mc_sparse(grid: SparseGrid, level: float, method: int, want_src: bool = False, want_jac: bool = False):
