@@ -696,7 +696,7 @@ __global__ void __launch_bounds__(64) k_dc_qef_grid(const int64_t *cell_dense, C
     if ((int64_t) blockIdx.x * 64 >= ncells) return;
     bool mine = a < ncells;
     if (mine && bt.items) {
-        // grids of one cell each are the rule in a wave: few steps, in the L2
+        // mostly all lanes of a wave are in one grid: few steps, the same loads
         int lo = 0, hi = bt.n;
         while (hi - lo > 1) {
             const int mid = (lo + hi) >> 1;
@@ -901,16 +901,6 @@ __global__ void k_dc_qef_prog(const int64_t *cell_dense, int64_t ncells, const C
 __constant__ const int8_t kNb[3][4][3] = {{{0, 0, 0}, {0, 1, 0}, {0, 1, 1}, {0, 0, 1}},
                                           {{0, 0, 0}, {0, 0, 1}, {1, 0, 1}, {1, 0, 0}},
                                           {{0, 0, 0}, {1, 0, 0}, {1, 1, 0}, {0, 1, 0}}};
-
-__device__ __forceinline__ int64_t lower_bound64(const int64_t *a, int64_t n, int64_t key) {
-    int64_t lo = 0, hi = n;
-    while (lo < hi) {
-        int64_t mid = (lo + hi) >> 1;
-        if (a[mid] < key) lo = mid + 1;
-        else hi = mid;
-    }
-    return lo;
-}
 
 // Active-cell hash: dense cell id -> active index (open addressing, linear
 // probing, at most half full).  Replaces a binary search per neighbour.
@@ -1581,8 +1571,6 @@ hipError_t fill_i64(int64_t *p, int64_t n, int64_t v, hipStream_t st) {
     return hipGetLastError();
 }
 
-// Launches the DC kernels (no synchronisation).  bt.items == nullptr: one
-// grid (s); otherwise the batch's grids.
 // Exclusive scan of nb block-sum pairs in place, totals to tot; part holds
 // dc_scan_part_pairs(nb) pairs.
 static void scan_pairs(int64_t *bsum, int64_t nb, int64_t *tot, int64_t *part, hipStream_t st) {
@@ -1625,6 +1613,8 @@ static void weld_and_emit(const CellSrc &s, const ItsIn &in, const CellCount &ce
         hipLaunchKernelGGL(k_remap_faces, dim3(nblocks(6 * in.npts)), dim3(kBlock), 0, st, w.tri_cells, w.tot, wd);
 }
 
+// Launches the DC kernels (no synchronisation).  bt.items == nullptr: one
+// grid (s); otherwise the batch's grids.
 static hipError_t dc_launch(const CellSrc &s, const ItsIn &in, float reg, float svd_tol, float cond_fp64,
                             DcScratch &w, const DcBatch &bt, hipStream_t st) {
     // Dense grids with lookup tables (the intersection set is the grid's

@@ -1780,11 +1780,6 @@ __global__ void mc_dense_reset(McParams p, SpecialLists init) {
     reset_state(p, init, (int64_t) blockIdx.x * blockDim.x + threadIdx.x, (int64_t) gridDim.x * blockDim.x);
 }
 
-// Concatenate the special-list segments (in segment order) into the
-// contiguous lists and record the counts and the capacity a call needs.
-// Workgroup b copies segment b of every list; its offset is the sum of the
-// (clamped) counts of the segments before it.
-static_assert(kSpSeg == 256, "sp_gather_seg maps one thread to each segment");
 // The call's read-back, by one thread of the last kernel; dup is written by
 // the duplicate check.
 __device__ __forceinline__ void host_result(const McParams &p, const unsigned long long n[4], unsigned long long need) {
@@ -1799,6 +1794,11 @@ __device__ __forceinline__ void host_result(const McParams &p, const unsigned lo
     h->sp.need = (int64_t) need;
 }
 
+// Concatenate the special-list segments (in segment order) into the
+// contiguous lists and record the counts and the capacity a call needs.
+// Workgroup b copies segment b of every list; its offset is the sum of the
+// (clamped) counts of the segments before it.
+static_assert(kSpSeg == 256, "sp_gather_seg maps one thread to each segment");
 __device__ __forceinline__ void sp_gather_seg(const McParams &p, int b) {
     // 256 threads, nseg <= 256: thread t reads segment t's four counters in
     // one round of loads; the offsets (clamped counts of the segments before
@@ -1869,8 +1869,6 @@ __device__ __forceinline__ void sp_gather_seg(const McParams &p, int b) {
         if (p.host) host_result(p, raw, nd);
     }
 }
-
-__global__ void __launch_bounds__(256) k_sp_gather(McParams p) { sp_gather_seg(p, blockIdx.x); }
 
 // Whether two gathered weld candidates share a position (as the fix-up
 // groups them: equal coordinates): candidate indices go into an
@@ -2431,7 +2429,8 @@ int64_t mc_config_tiles(int cfg, const int64_t shape[3]) {
 // 82.5, 192^3 84.3 -> 92.9.  Thin tiles, noise: 120x120x6 (320 cells) 73.2 ->
 // 69.9, 120x120x5 (256) 55.3 -> 56.7, 300x300x2 76.6 -> 106.9.  The tiles of
 // an intersection pass alone (8 spheres): 64^3 25.6 -> 19.4, 128^3 28.6 ->
-// 21.4 us.  128 threads a tile: 64^3 45.1 instead of 45.5 us, 160^3 61.9
+// 21.4 us (a set of noise, where every cell crosses: 445 -> 503 the whole call
+// at 128^3).  128 threads a tile: 64^3 45.1 instead of 45.5 us, 160^3 61.9
 // instead of 60.0; 64 threads 51.5 at 64^3.
 int mc_auto_config(const int64_t shape[3]) {
     static const int order[] = {3, 1, 5};
