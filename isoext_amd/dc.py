@@ -230,10 +230,12 @@ def _remember(hints, shape, sizes, low=None):
     for, a large surface still fits after three small ones of its shape (too
     little room costs a second run), and a lone large one is soon forgotten.
     low: the last size from the other side, an eighth of the way a call."""
+    if hints.get(shape) == sizes and (low is None or low.get(shape) == sizes[-1]):
+        return   # nothing changes: no lock
     with _hint_lock:
         if len(hints) > 4096:
             hints.clear()
-        hints[shape] = tuple(max(n, o - o // 32) for n, o in zip(sizes, hints.get(shape, sizes)))
+        hints[shape] = tuple([max(n, o - o // 32) for n, o in zip(sizes, hints.get(shape, sizes))])
         if low is not None:
             if len(low) > 4096:
                 low.clear()
@@ -245,8 +247,8 @@ def _its_vary(shape):
     """Whether a shape's recent intersection sets differ so much that room for
     the largest would mean copying the others out of it (eight copies, 40 us,
     where waiting for the count before the buffers are made takes 20)."""
-    low = _its_low.get(shape)
-    return low is not None and shape in _its_hint and _its_caps(shape)[1] > 2 * low + _PINNED
+    hint, low = _its_hint.get(shape), _its_low.get(shape)
+    return hint is not None and low is not None and hint[1] + (hint[1] >> 3) + 4096 > 2 * low + _PINNED
 
 
 # Most cells that a call without a hint makes room for; a call that needs more
@@ -255,10 +257,8 @@ _FIRST_CELLS = 1 << 22
 
 
 def _most_cells(shape):
-    n = 1
-    for s in shape:
-        n *= max(int(s) - 1, 0)
-    return max(n, 1)
+    X, Y, Z = shape
+    return (X - 1) * (Y - 1) * (Z - 1) if X > 1 and Y > 1 and Z > 1 else 1
 
 
 def _first_cells(shape):
@@ -268,12 +268,13 @@ def _first_cells(shape):
 
 
 def _its_caps(shape):
-    most = min(_most_cells(shape), 0x7fffffff)
     hint = _its_hint.get(shape)   # a single dict read needs no lock
     if hint is None:
         cells = _first_cells(shape)
         return cells, 4 * cells
-    return min(hint[0] + hint[0] // 8 + 1024, most), min(hint[1] + hint[1] // 8 + 4096, 12 * most)
+    c, p = hint
+    most = min(_most_cells(shape), 0x7fffffff)
+    return min(c + (c >> 3) + 1024, most), min(p + (p >> 3) + 4096, 12 * most)
 
 
 def _dc_caps(shape):
@@ -281,8 +282,9 @@ def _dc_caps(shape):
     if hint is None:
         nc = _first_cells(shape)
         return nc, nc, 2 * nc
+    c, v, f = hint
     most = min(_most_cells(shape), 0x3fffffff)
-    return tuple(min(n + n // 8 + 1024, k * most) for n, k in zip(hint, (1, 1, 6)))
+    return min(c + (c >> 3) + 1024, most), min(v + (v >> 3) + 1024, most), min(f + (f >> 3) + 1024, 6 * most)
 
 
 def _its_buffers(nc, npt, normals, dev):
@@ -401,13 +403,13 @@ def _dc_grid(grid, level: float, reg: float, svd_tol: float):
             else:
                 cap_v, cap_f = max(cap_v, int(counts[0])), max(cap_f, int(counts[1]))
     _lib.check(rc, "dual_contouring")
-    nv, nf = int(counts[0]), int(counts[1])
-    _remember(_dc_hint, shape, (int(counts[3]), nv, nf))
-    if (shape in _dc_none) != (counts[3] == 0):
+    nv, nf, _, cells, _ = counts
+    _remember(_dc_hint, shape, (cells, nv, nf))
+    if (shape in _dc_none) != (cells == 0):
         with _hint_lock:
             if len(_dc_none) > 4096:
                 _dc_none.clear()
-            (_dc_none.discard if counts[3] else _dc_none.add)(shape)
+            (_dc_none.discard if cells else _dc_none.add)(shape)
     if nf == 0:
         return None, None
     v, f = out_v[:nv], out_f[:nf]
