@@ -211,7 +211,8 @@ int isoext_dc(const isoext_grid *g, const isoext_its *its, float reg, float svd_
  * stream, grid, level and scratch) launches the rest into buffers of
  * cap_cells (cell_offsets: cap_cells + 1) and cap_pts entries and waits for
  * the counts only, {cells, points}.  On ISOEXT_E_CAPACITY they hold the need,
- * and finish may be called again with more room. */
+ * and finish may be called again with more room.  A set that was begun and
+ * given up is waited for by the thread's next begin. */
 int isoext_its_begin(const isoext_grid *g, float level, void *scratch, int64_t scratch_bytes, void *stream);
 int isoext_its_finish(const isoext_grid *g, float level, void *scratch, int64_t cap_cells, int64_t cap_pts,
                       int64_t *cell_indices, int64_t *cell_dense, int64_t *cell_offsets, float *points,
