@@ -80,7 +80,9 @@ int64_t isoext_mc_dense_workspace_bytes(const int64_t shape[3], int cfg, int64_t
  * src/isoext_ext.cu:95-109.  method: 0 = "nagae", 1 = "lorensen"
  * (src/mc/base.cu:19-27).  Writes up to cap_v vertices (3 floats each) and
  * cap_f faces (3 int32 each).  counts[0..1] = vertices, faces of the final
- * mesh; counts[2] = special-list capacity needed; counts[3] = device error
+ * mesh; counts[2] = special-list capacity needed (of the fullest list segment,
+ * about a percent up or down from run to run: leave some room when a call is
+ * repeated, isoext_amd.mc takes an eighth); counts[3] = device error
  * bits; counts[4..5] = provisional vertices, faces (before the weld fix-up
  * removes duplicates): the capacities a call on the same input needs.  On
  * ISOEXT_E_CAPACITY counts[0..1] also hold the provisional sizes to allocate
